@@ -362,6 +362,21 @@ int jmm_pair_observables(const jmm_chain_spec *spec, int n_configs, const double
                          const double *L_dev, double *obs_dev, double *grad_dev, int precision,
                          void *stream);
 
+/* jmm_pair_observables with a work array: *work_doubles = how many doubles
+ * of device memory spread n_configs configurations of this spec over the
+ * whole GPU (0: short configurations, which need none). */
+int jmm_pair_observables_work(const jmm_chain_spec *spec, int n_configs, uint64_t *work_doubles);
+
+/* As jmm_pair_observables, with work_dev[work_doubles] in DEVICE memory that
+ * is free until the call's work on the stream is done (contents do not
+ * matter).  A NULL or smaller array runs one workgroup per configuration, as
+ * jmm_pair_observables does; the sums over a configuration's pairs are then
+ * taken in another order.  Asynchronous on the stream, allocates nothing.  No
+ * reference counterpart. */
+int jmm_pair_observables_ws(const jmm_chain_spec *spec, int n_configs, const double *x_dev,
+                            const double *L_dev, double *obs_dev, double *grad_dev, int precision,
+                            void *stream, double *work_dev, uint64_t work_doubles);
+
 #ifdef __cplusplus
 }
 #endif

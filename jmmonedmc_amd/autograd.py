@@ -19,7 +19,7 @@ import dataclasses
 import numpy as np
 import torch
 
-from .engine import Chain, pair_observables
+from .engine import Chain, pair_observables, pair_observables_work
 
 
 def _observables(x: torch.Tensor, L: torch.Tensor, chain: Chain, theta, precision: int,
@@ -34,12 +34,17 @@ def _observables(x: torch.Tensor, L: torch.Tensor, chain: Chain, theta, precisio
     th = [float(t) for t in theta]
     p = list(chain.pot_p) + [0.0] * (4 - len(chain.pot_p))
     p[0], p[1] = th[0], th[1]
-    ch = dataclasses.replace(chain, N=N, pot_p=tuple(p), L0=float(L[0].item()) if n else 1.0)
+    # the kernel reads each configuration's length from L: the chain's own is
+    # not used (and not copied back from the device for it)
+    ch = dataclasses.replace(chain, N=N, pot_p=tuple(p), L0=1.0)
     obs = torch.empty((n, 6), dtype=torch.float64, device=x.device)
     grad = torch.empty_like(x) if want_grad else None
     stream = torch.cuda.current_stream(x.device).cuda_stream
+    nw = pair_observables_work(ch, n) if n else 0
+    work = torch.empty(nw, dtype=torch.float64, device=x.device) if nw else None
     pair_observables(ch, x.data_ptr(), L.data_ptr(), obs.data_ptr(),
-                     grad.data_ptr() if want_grad else None, n, precision, stream)
+                     grad.data_ptr() if want_grad else None, n, precision, stream,
+                     work.data_ptr() if nw else None, nw)
     return obs, grad
 
 

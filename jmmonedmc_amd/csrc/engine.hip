@@ -290,8 +290,13 @@ struct jmm_engine {
     uint32_t *d_ext = nullptr;      // external index of each internal chain
     uint64_t *d_extoff = nullptr;   // external position offset of each internal chain
     uint8_t *d_log = nullptr;
-    double *d_obs = nullptr, *d_grad = nullptr, *d_Ltmp = nullptr, *d_Lnew = nullptr;
-    uint32_t *d_all = nullptr;
+    double *d_obs = nullptr, *d_grad = nullptr, *d_Lnew = nullptr;
+    // observables kernel: tiles of long chains, their partial sums
+    ObsTile *d_tiles = nullptr;
+    uint32_t *d_first = nullptr;
+    double *d_obs_part = nullptr;
+    uint32_t obs_tiles = 0;
+    int obs_threads = 256;
     uint32_t cap = 1024, write_pos = 0, block_sweeps = 100;
     std::vector<Group> grp;
     int use_graph = 0;
@@ -554,9 +559,10 @@ int jmm_destroy(jmm_engine *e)
     (void)hipFree(e->d_log);
     (void)hipFree(e->d_obs);
     (void)hipFree(e->d_grad);
-    (void)hipFree(e->d_Ltmp);
     (void)hipFree(e->d_Lnew);
-    (void)hipFree(e->d_all);
+    (void)hipFree(e->d_tiles);
+    (void)hipFree(e->d_first);
+    (void)hipFree(e->d_obs_part);
     (void)hipFree(e->d_rho);
     (void)hipFree(e->d_g);
     (void)hipFree(e->d_packed);
@@ -1335,6 +1341,38 @@ int jmm_get_counters(jmm_engine *e, int chain, jmm_counters *out)
     return 0;
 }
 
+// Tiles of every chain for the observables kernel (chains longer than
+// OBS_ONE; otherwise one workgroup each, and only the buffers).
+static int ensure_obs(jmm_engine *e)
+{
+    if (e->d_obs) return 0;
+    uint32_t nmax = 1;
+    for (const auto &c : e->hch) nmax = std::max(nmax, c.N);
+    if (nmax > OBS_ONE && !e->obs_tiles) {
+        std::vector<ObsTile> tiles;
+        std::vector<uint32_t> first(1, 0u);
+        for (uint32_t k = 0; k < (uint32_t)e->n; ++k) {
+            for (uint32_t p = 0; p * OBS_TILE < e->hch[k].N; ++p) tiles.push_back({k, p});
+            first.push_back((uint32_t)tiles.size());
+        }
+        // (an attempt that ran out of memory half-way kept what it had)
+        if (!e->d_tiles)
+            if (int rc = dalloc(&e->d_tiles, tiles.size())) return rc;
+        if (!e->d_first)
+            if (int rc = dalloc(&e->d_first, first.size())) return rc;
+        if (!e->d_obs_part)
+            if (int rc = dalloc(&e->d_obs_part, tiles.size() * 6)) return rc;
+        HIPCHK(hipMemcpy(e->d_tiles, tiles.data(), sizeof(ObsTile) * tiles.size(), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(e->d_first, first.data(), sizeof(uint32_t) * first.size(), hipMemcpyHostToDevice));
+        e->obs_tiles = (uint32_t)tiles.size();
+        e->obs_threads = (int)OBS_TILE;
+    } else if (nmax <= OBS_ONE) {
+        e->obs_tiles = (uint32_t)e->n;
+        e->obs_threads = (int)((nmax + 63) / 64 * 64);
+    }
+    return dalloc(&e->d_obs, (size_t)e->n * 6);
+}
+
 // obs/grad: host arrays (copied out after the kernel, synchronous), or with
 // on_device the caller's device arrays, written by the kernel on the
 // engine's stream and not waited for.
@@ -1343,33 +1381,25 @@ static int observables_impl(jmm_engine *e, double *obs, double *grad, int fp32,
 {
     HIPCHK(hipSetDevice(e->device));
     if (int rc = ensure_ext(e)) return rc;
-    if (!e->d_obs)
-        if (int rc = dalloc(&e->d_obs, (size_t)e->n * 6)) return rc;
-    if (!e->d_Ltmp)
-        if (int rc = dalloc(&e->d_Ltmp, (size_t)e->n)) return rc;
-    if (!e->d_all) {
-        if (int rc = dalloc(&e->d_all, (size_t)e->n)) return rc;
-        std::vector<uint32_t> all(e->n);
-        std::iota(all.begin(), all.end(), 0u);
-        HIPCHK(hipMemcpy(e->d_all, all.data(), sizeof(uint32_t) * e->n, hipMemcpyHostToDevice));
-    }
+    if (int rc = ensure_obs(e)) return rc;
     if (grad && !on_device && !e->d_grad)
         if (int rc = dalloc(&e->d_grad, e->total_N)) return rc;
-    HIPCHK(launch_lengths(e->d_states, e->d_Ltmp, (uint32_t)e->n, e->stream));
     ObsArgs a{};
     a.chains = e->d_chains;
+    a.states = e->d_states;
     a.x = e->d_x;
-    a.L = e->d_Ltmp;
-    a.list = e->d_all;
     a.Lnew = Lnew_dev;
+    a.tiles = e->d_tiles;
+    a.first = e->d_first;
+    a.part = e->d_obs_part;
+    a.tile = e->d_tiles ? OBS_TILE : OBS_ONE;
+    a.parts = 1;
     a.obs = on_device ? obs : e->d_obs;
     a.grad = on_device ? grad : (grad ? e->d_grad : nullptr);
     // results in the caller's chain order, copied out as they are
     a.row = e->d_ext;
     a.goff = e->d_extoff;
-    a.n = (uint32_t)e->n;
-    a.standalone = 0;
-    HIPCHK(launch_observables(a, fp32, (uint32_t)e->n, e->stream));
+    HIPCHK(launch_observables(a, fp32, e->obs_tiles, (uint32_t)e->n, e->obs_threads, e->stream));
     if (on_device) return 0;
     HIPCHK(hipStreamSynchronize(e->stream));
     HIPCHK(hipMemcpy(obs, e->d_obs, sizeof(double) * (size_t)e->n * 6, hipMemcpyDeviceToHost));
@@ -1481,9 +1511,31 @@ int jmm_full_energy(jmm_engine *e, double *U_out)
     return 0;
 }
 
+// Workgroups per configuration of the standalone form.
+static uint32_t obs_parts(uint64_t N)
+{
+    return N <= OBS_ONE ? 1u : (uint32_t)((N + OBS_TILE - 1) / OBS_TILE);
+}
+
+int jmm_pair_observables_work(const jmm_chain_spec *spec, int n_configs, uint64_t *work_doubles)
+{
+    if (!spec || n_configs <= 0 || !work_doubles)
+        return fail(JMM_EINVAL, "jmm_pair_observables_work: null or empty argument");
+    const uint64_t parts = obs_parts(spec->N);
+    *work_doubles = parts > 1 ? parts * 6 * (uint64_t)n_configs : 0;
+    return 0;
+}
+
 int jmm_pair_observables(const jmm_chain_spec *spec, int n_configs, const double *x_dev,
                          const double *L_dev, double *obs_dev, double *grad_dev, int precision,
                          void *stream)
+{
+    return jmm_pair_observables_ws(spec, n_configs, x_dev, L_dev, obs_dev, grad_dev, precision, stream, nullptr, 0);
+}
+
+int jmm_pair_observables_ws(const jmm_chain_spec *spec, int n_configs, const double *x_dev,
+                            const double *L_dev, double *obs_dev, double *grad_dev, int precision,
+                            void *stream, double *work_dev, uint64_t work_doubles)
 {
     if (!spec || n_configs <= 0 || !x_dev || !L_dev || !obs_dev)
         return fail(JMM_EINVAL, "jmm_pair_observables: null or empty argument");
@@ -1501,9 +1553,22 @@ int jmm_pair_observables(const jmm_chain_spec *spec, int n_configs, const double
     a.L = L_dev;
     a.obs = obs_dev;
     a.grad = grad_dev;
-    a.n = (uint32_t)n_configs;
     a.standalone = 1;
-    HIPCHK(launch_observables(a, precision == 32, (uint32_t)n_configs, (hipStream_t)stream));
+    // long configurations: tiles over the chip where the caller's work array
+    // holds their partial sums, else one workgroup each
+    const uint64_t parts = obs_parts(s.N);
+    if (parts > 1 && work_dev && work_doubles >= parts * 6 * (uint64_t)n_configs &&
+        parts * (uint64_t)n_configs <= 0x7fffffffull) {
+        a.parts = (uint32_t)parts;
+        a.tile = OBS_TILE;
+        a.part = work_dev;
+    } else {
+        a.parts = 1;
+        a.tile = a.one.N;
+    }
+    const int threads = a.part ? (int)OBS_TILE : (int)std::min<uint64_t>(OBS_ONE, (s.N + 63) / 64 * 64);
+    HIPCHK(launch_observables(a, precision == 32, a.parts * (uint32_t)n_configs, (uint32_t)n_configs, threads,
+                              (hipStream_t)stream));
     return 0;
 }
 

@@ -83,18 +83,32 @@ struct SweepArgs {
     uint32_t n_items, n_sweeps, n_chains, cap;
 };
 
+// A tile of a configuration: particles [part * OBS_TILE, (part + 1) * OBS_TILE).
+struct ObsTile {
+    uint32_t chain, part;
+};
+
+// Configurations of up to OBS_ONE particles are one workgroup's (a particle
+// per lane, nothing to add afterwards); longer ones are cut into tiles of
+// OBS_TILE, summed by a second launch (about 3 us, against 30 us saved per
+// 1024 particles of a configuration that one workgroup walks in turn).
+constexpr uint32_t OBS_ONE = 1024, OBS_TILE = 256;
+
 struct ObsArgs {
     const DevChain *chains;  // engine form (nullable)
+    const DevState *states;  // engine form: the chains' lengths
     DevChain one;            // standalone form
     const double *x;
-    const double *L;
-    const uint32_t *list;    // engine form: chains of this launch
+    const double *L;         // standalone form
+    const ObsTile *tiles;    // engine form, nullable: tiles of all chains in chain order
+    const uint32_t *first;   // engine form with tiles: [n + 1], first tile of each chain
     const double *Lnew;      // engine form, nullable: evaluate at x * Lnew/L, length Lnew
+    double *part;            // nullable: [tile][6] partial sums, for k_obs_sum
     double *obs;
     double *grad;
     const uint32_t *row;     // engine form, nullable: output row of each chain (else its index)
     const uint64_t *goff;    // engine form, nullable: gradient offset of each chain (else x_off)
-    uint32_t n;
+    uint32_t tile, parts;    // particles per workgroup; standalone form: workgroups per configuration
     uint32_t standalone;
 };
 
@@ -144,8 +158,8 @@ hipError_t launch_batched(const SweepArgs &a, int fp32, int T, int gx, uint32_t 
                           hipStream_t s);
 const void *plain_kernel(int gx);
 hipError_t launch_plain(const SweepArgs &a, int gx, uint32_t grid, size_t lds, hipStream_t s);
-hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t grid, hipStream_t s);
-hipError_t launch_lengths(const DevState *st, double *L, uint32_t n, hipStream_t s);
+hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads,
+                              hipStream_t s);
 // Samples in the caller's layout (jmm_sample): out[ext[k] * n_sweeps + s]
 // from the engine's [sweep][chain] arrays.
 struct SampleRec {

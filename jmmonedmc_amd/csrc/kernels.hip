@@ -12,7 +12,8 @@
 //                    energy change a wavefront reduction over the neighbour
 //                    window (lanes 0-31 left partners, 32-63 right).
 //   k_observables    U, virial, dU/dtheta, dW/dtheta and dU/dx per
-//                    configuration (the differentiation path).
+//                    configuration (the differentiation path), one workgroup
+//                    per tile of a configuration; k_obs_sum adds the tiles.
 //   k_begin          resets a work queue and advances the sample row.
 #include "kernels.h"
 
@@ -1906,39 +1907,48 @@ __global__ void k_begin(Ctrl *c, uint32_t n)
 
 // ------------------------------------------------------- differentiation
 
-// One workgroup per configuration.  Pair arithmetic in Real, sums in FP64.
-// obs = (U, W, dU/dtheta0, dU/dtheta1, dW/dtheta0, dW/dtheta1); grad = dU/dx.
+// U, W and their parameter derivatives of one tile of a configuration
+// (particles [p0, p1): the pairs whose left member is in the tile) and dU/dx
+// of the tile's particles.  Pair arithmetic in Real, sums in FP64.
+// out = (U, W, dU/dtheta0, dU/dtheta1, dW/dtheta0, dW/dtheta1) of the tile.
+//
+// Bound by vector issue: about 16 pairs a side for the 20 sigma Yukawa
+// chains at density 0.8, each some 70 instructions (an FP32 exponential and
+// division or an FP64 division, and six FP64 sums) against 16 bytes of
+// memory per particle, so what matters is that every SIMD has waves to
+// issue from.  A particle per lane and tiles of OBS_TILE spread a long
+// configuration over the chip, where one workgroup each left 64
+// configurations of 65,536 on 64 of the 256 CUs with one wave per SIMD
+// (forward and backward of those through the autograd binding, FP32: 3.67 ms
+// with one workgroup each, 0.376 ms with tiles).
+// Neighbouring lanes read neighbouring positions (L1 hits); the left partners
+// are evaluated again for dU/dx (W only) rather than exchanged, which would
+// need a barrier per partner.
 template <typename Real, int KIND>
-__device__ void run_obs(const DevChain &ch, const double *X, double L, double sc, double *obs,
-                        double *grad)
+__device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, double L, double sc, uint32_t p0,
+                                        uint32_t p1, double *out, double *grad)
 {
-    __shared__ double red[4 * 6];
+    __shared__ double red[16 * 6];
     const uint32_t tid = threadIdx.x;
     const Pot q = ch.pot;
-    const int64_t N = ch.N;
+    const uint32_t N = ch.N;
     // a compressed configuration (sc < 1) may hold gaps below the hard core:
     // walk to the cutoff (or the NBN limit) without the window limit
-    const uint32_t w = sc < 1.0 ? min(ch.nbn_lim, (uint32_t)(N > 0 ? N - 1 : 0)) : ch.w;
+    const uint32_t w = sc < 1.0 ? min(ch.nbn_lim, N > 0 ? N - 1 : 0u) : ch.w;
     const bool per = (ch.flags & F_PERIODIC) != 0;
     const Real sh[3] = {Real(ch.sh[0]), Real(ch.sh[1]), Real(ch.sh[2])};
-    // position j (index possibly past either end on a periodic line) of the
-    // configuration scaled by sc to length L: x_j sc, images x sc -+ L
-    auto pos = [&](int64_t j, double &xj) -> bool {
-        if (j >= 0 && j < N) {
-            xj = X[j] * sc;
-            return true;
-        }
-        if (!per) return false;
-        xj = (j < 0) ? X[j + N] * sc - L : X[j - N] * sc + L;
-        return true;
-    };
     double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (uint32_t i = tid; i < (uint32_t)N; i += 256) {
+    for (uint32_t i = p0 + tid; i < p1; i += blockDim.x) {
+        // positions of the configuration scaled by sc to length L: x_j sc,
+        // periodic images x_j sc -+ L
         const double xi = X[i] * sc;
         double g = 0.0;
         for (uint32_t k = 1; k <= w; ++k) {
+            const uint32_t j = i + k;
             double xj;
-            if (!pos((int64_t)i + k, xj)) break;
+            if (j < N) xj = X[j] * sc;
+            else if (per) xj = X[j - N] * sc + L;
+            else break;
             const double d = xj - xi;
             if (d > q.rc) break;
             // a rescaled configuration can overlap hard cores: infinite energy
@@ -1956,7 +1966,9 @@ __device__ void run_obs(const DevChain &ch, const double *X, double L, double sc
         if (grad) {
             for (uint32_t k = 1; k <= w; ++k) {
                 double xj;
-                if (!pos((int64_t)i - k, xj)) break;
+                if (k <= i) xj = X[i - k] * sc;
+                else if (per) xj = X[i + N - k] * sc - L;
+                else break;
                 const double d = xi - xj;
                 if (d > q.rc) break;
                 if (!inside64<KIND>(q, d)) continue;
@@ -1972,49 +1984,74 @@ __device__ void run_obs(const DevChain &ch, const double *X, double L, double sc
     if ((tid & 63) == 0)
         for (int m = 0; m < 6; ++m) red[(tid >> 6) * 6 + m] = acc[m];
     __syncthreads();
-    if (tid == 0)
-        for (int m = 0; m < 6; ++m) obs[m] = ((red[m] + red[6 + m]) + red[12 + m]) + red[18 + m];
+    if (tid < 6) {
+        double v = 0.0;
+        for (uint32_t wv = 0; wv < (blockDim.x >> 6); ++wv) v += red[wv * 6 + tid];
+        out[tid] = v;
+    }
 }
 
+// One workgroup per tile: a.tile particles of a configuration, or the whole
+// configuration (a.tiles = nullptr), whose observables then go straight to
+// the caller's row; with tiles they go to a.part, and k_obs_sum adds them.
 template <typename Real>
-__global__ void __launch_bounds__(256) k_observables(ObsArgs a)
+__global__ void __launch_bounds__(1024) k_observables(ObsArgs a)
 {
-    const uint32_t c = blockIdx.x;
-    const DevChain &ch = a.standalone ? a.one : a.chains[a.list[c]];
+    uint32_t c, p0 = 0, part = 0;
+    if (a.standalone) {
+        c = blockIdx.x / a.parts;
+        part = blockIdx.x % a.parts;
+    } else if (a.tiles) {
+        c = a.tiles[blockIdx.x].chain;
+        part = a.tiles[blockIdx.x].part;
+    } else {
+        c = blockIdx.x;
+    }
+    const DevChain &ch = a.standalone ? a.one : a.chains[c];
+    const uint32_t N = ch.N;
+    p0 = part * a.tile;
+    const uint32_t p1 = min(N, p0 + a.tile);
     const double *X;
-    double L, *grad;
-    double *obs;
+    double L, *grad, *out;
     double sc = 1.0;
     if (a.standalone) {
-        X = a.x + (uint64_t)c * ch.N;
+        X = a.x + (uint64_t)c * N;
         L = a.L[c];
-        grad = a.grad ? a.grad + (uint64_t)c * ch.N : nullptr;
-        obs = a.obs + (uint64_t)c * 6;
+        grad = a.grad ? a.grad + (uint64_t)c * N : nullptr;
     } else {
-        const uint32_t ic = a.list[c];
         X = a.x + ch.x_off;
-        L = a.L[ic];
+        L = a.states[c].L;
         if (a.Lnew) {
-            sc = a.Lnew[ic] / L;
-            L = a.Lnew[ic];
+            sc = a.Lnew[c] / L;
+            L = a.Lnew[c];
         }
-        grad = a.grad ? a.grad + (a.goff ? a.goff[ic] : ch.x_off) : nullptr;
-        obs = a.obs + (uint64_t)(a.row ? a.row[ic] : ic) * 6;
+        grad = a.grad ? a.grad + (a.goff ? a.goff[c] : ch.x_off) : nullptr;
     }
+    if (a.part) out = a.part + (uint64_t)blockIdx.x * 6;
+    else out = a.obs + (uint64_t)(a.row ? a.row[c] : c) * 6;
     switch (ch.kind) {
-    case POT_LJ: run_obs<Real, POT_LJ>(ch, X, L, sc, obs, grad); break;
-    case POT_HARMONIC: run_obs<Real, POT_HARMONIC>(ch, X, L, sc, obs, grad); break;
-    case POT_HRSW: run_obs<Real, POT_HRSW>(ch, X, L, sc, obs, grad); break;
-    default: run_obs<Real, POT_YUKAWA>(ch, X, L, sc, obs, grad); break;
+    case POT_LJ: run_obs<Real, POT_LJ>(ch, X, L, sc, p0, p1, out, grad); break;
+    case POT_HARMONIC: run_obs<Real, POT_HARMONIC>(ch, X, L, sc, p0, p1, out, grad); break;
+    case POT_HRSW: run_obs<Real, POT_HRSW>(ch, X, L, sc, p0, p1, out, grad); break;
+    default: run_obs<Real, POT_YUKAWA>(ch, X, L, sc, p0, p1, out, grad); break;
     }
 }
 
-// Copies every chain's current length out of the state array (observables
-// of engine chains).
-__global__ void k_lengths(const DevState *st, double *L, uint32_t n)
+// Sums each configuration's tiles: lanes stride over the tiles, then a wave
+// sum per field (a fixed order, the same on every call).
+__global__ void __launch_bounds__(64) k_obs_sum(ObsArgs a)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) L[i] = st[i].L;
+    const uint32_t c = blockIdx.x, lane = threadIdx.x;
+    const uint32_t first = a.standalone ? c * a.parts : a.first[c];
+    const uint32_t n = a.standalone ? a.parts : a.first[c + 1] - first;
+    double v[6] = {0, 0, 0, 0, 0, 0};
+    for (uint32_t p = lane; p < n; p += 64)
+        for (int m = 0; m < 6; ++m) v[m] += a.part[(uint64_t)(first + p) * 6 + m];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) v[m] = wave_sum(v[m]);
+    double *o = a.obs + (uint64_t)(a.row ? a.row[c] : c) * 6;
+    if (lane == 0)
+        for (int m = 0; m < 6; ++m) o[m] = v[m];
 }
 
 // Sample rows [sweep][chain] (internal chain order) to the caller's layout
@@ -2204,10 +2241,12 @@ hipError_t launch_plain(const SweepArgs &a, int gx, uint32_t grid, size_t lds, h
     return hipGetLastError();
 }
 
-hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t grid, hipStream_t s)
+hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads,
+                              hipStream_t s)
 {
-    if (fp32) hipLaunchKernelGGL(k_observables<float>, dim3(grid), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(k_observables<double>, dim3(grid), dim3(256), 0, s, a);
+    if (fp32) hipLaunchKernelGGL(k_observables<float>, dim3(n_tiles), dim3(threads), 0, s, a);
+    else hipLaunchKernelGGL(k_observables<double>, dim3(n_tiles), dim3(threads), 0, s, a);
+    if (a.part) hipLaunchKernelGGL(k_obs_sum, dim3(n_configs), dim3(64), 0, s, a);
     return hipGetLastError();
 }
 
@@ -2244,12 +2283,6 @@ hipError_t launch_segmented(const SegArgs &a, int fp32, int tw, int lpb, size_t 
 hipError_t launch_hist(const HistArgs &a, hipStream_t s)
 {
     hipLaunchKernelGGL(k_hist, dim3(a.n_chains * a.parts), dim3(256), 0, s, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_lengths(const DevState *st, double *L, uint32_t n, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_lengths, dim3((n + 255) / 256), dim3(256), 0, s, st, L, n);
     return hipGetLastError();
 }
 

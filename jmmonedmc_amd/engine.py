@@ -284,12 +284,22 @@ class Engine:
         return n.value, ms.value, sw.value
 
 
+def pair_observables_work(chain: Chain, n_configs: int) -> int:
+    """Doubles of device memory with which pair_observables spreads these
+    configurations over the whole GPU (0: it needs none)."""
+    s, n = chain.to_c(), C.c_uint64()
+    check(lib().jmm_pair_observables_work(C.byref(s), n_configs, C.byref(n)), "jmm_pair_observables_work")
+    return n.value
+
+
 def pair_observables(chain: Chain, x_ptr: int, L_ptr: int, obs_ptr: int, grad_ptr: int | None,
-                     n_configs: int, precision: int = 64, stream: int | None = None):
+                     n_configs: int, precision: int = 64, stream: int | None = None,
+                     work_ptr: int | None = None, work_doubles: int = 0):
     """Backward kernel on caller-owned device memory (raw pointers)."""
     s = chain.to_c()
-    check(lib().jmm_pair_observables(C.byref(s), n_configs, C.c_void_p(x_ptr), C.c_void_p(L_ptr),
-                                     C.c_void_p(obs_ptr),
-                                     C.c_void_p(grad_ptr) if grad_ptr else None, precision,
-                                     C.c_void_p(stream) if stream else None),
+    check(lib().jmm_pair_observables_ws(C.byref(s), n_configs, C.c_void_p(x_ptr), C.c_void_p(L_ptr),
+                                        C.c_void_p(obs_ptr),
+                                        C.c_void_p(grad_ptr) if grad_ptr else None, precision,
+                                        C.c_void_p(stream) if stream else None,
+                                        C.c_void_p(work_ptr) if work_ptr else None, work_doubles),
           "jmm_pair_observables")
