@@ -833,7 +833,7 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
         if (!segv.empty()) {
             const int fp32 = e->form == JMM_FORM_BATCHED_FP32;
             if (o.seg_lanes > 2) return bail(fail(JMM_EINVAL, "jmm_create: seg_lanes must be 0, 1 or 2"));
-            e->seg_lpb = o.seg_lanes ? (int)o.seg_lanes : 1;
+            e->seg_lpb = o.seg_lanes ? (int)o.seg_lanes : (fp32 ? 2 : 1);
             e->seg_tw = e->seg_lpb * bsmax > 256 ? 512 : 256;
             for (int c = 0; c < n_chains; ++c)
                 if (segS[c]) e->layout[c].lanes = (uint32_t)e->seg_lpb;

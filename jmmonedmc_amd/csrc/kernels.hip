@@ -604,6 +604,87 @@ __device__ __forceinline__ bool walk_in(const Pot &, double, double, bool io, bo
     return io || in;
 }
 
+// Energy change of one side's partners, FP32 form, for two lanes per block:
+// the lane walks the partners at my - k (left) or my + k (right), four per
+// loop iteration, and returns the sum of their FP32 terms in FP64, added in
+// the order k = 1, 2, ... as the one-lane walk adds that side's.  The
+// positions are sorted, so the separations grow with k and a partner outside
+// the cutoff at both positions is followed by none inside: the FP64
+// inside-the-cutoff flags alone make the later terms zero, and the walk needs
+// no liveness or per-lane limit beyond them (w, the same on every lane, ends
+// the loop; a chain with walls holds NaN where it has no partner, which is
+// inside nothing).  |x| replaces the side's orientation of a separation
+// (xj - xi is -(xi - xj) exactly; a trial that goes on keeps the sign of the
+// new separation by the hard-core test).  A lane whose trial is already
+// rejected walks with the others and its result is dropped.
+//
+// Bound by vector issue: per partner 2 quarter-rate instructions per pair
+// energy for Yukawa (exponential, reciprocal) and about 30 others.  Eight
+// independent pair energies per iteration keep one wave issuing; the walk of
+// one partner per iteration, with liveness, was latency-bound.  With it and
+// the shared box-length pass two lanes per block (two waves per SIMD, VALU
+// busy 74 %) run 50 sweeps of 64 chains of 65,536 in 16.9 ms, one lane per
+// block (one wave, 56 %) in 20.1.
+template <int KIND>
+__device__ __forceinline__ double walk_side32(const double *X, const Pot &q, uint32_t w, bool go, bool left,
+                                              uint32_t t, uint32_t size, uint32_t my, uint32_t gapL, uint32_t gapR,
+                                              double xi, double xn, uint32_t &terms)
+{
+    const uint32_t m = left ? t : size - 1 - t;           // partners of the own block on this side
+    const uint32_t gap = (left ? 0u - gapL : gapR) * 8u;  // bytes to the next block's, modulo 2^32
+    const uint32_t dir = left ? 0u - 8u : 8u;
+    const uint32_t at = my * 8u;
+    const char *XB = (const char *)X;
+    double sum = 0.0;
+    int well = 0;
+    uint32_t cnt = 0;
+    bool more = go;
+    auto step = [&](uint32_t k, double &o, double &n) {
+        const double xj = *(const double *)(XB + (at + dir * k + (k > m ? gap : 0u)));
+        o = fabs(xi - xj);
+        n = fabs(xn - xj);
+    };
+    auto term = [&](double o, double n, bool io, bool in) -> float {
+        return phi32<KIND>(q, (float)n, in) - phi32<KIND>(q, (float)o, io);
+    };
+    uint32_t k = 1;
+    while (k + 3 <= w && __any(more)) {
+        double o[4], n[4];
+        bool io[4], in[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            step(k + u, o[u], n[u]);
+            io[u] = inside64<KIND>(q, o[u]);
+            in[u] = inside64<KIND>(q, n[u]);
+            cnt += (io[u] ? 1u : 0u) + (in[u] ? 1u : 0u);
+        }
+        if (KIND == POT_HRSW) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) well += (int)in[u] - (int)io[u];
+        } else {
+            float e[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) e[u] = term(o[u], n[u], io[u], in[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) sum += (double)e[u];
+        }
+        more = go && (io[3] || in[3]);
+        k += 4;
+    }
+    while (k <= w && __any(more)) {
+        double o, n;
+        step(k, o, n);
+        const bool io = inside64<KIND>(q, o), in = inside64<KIND>(q, n);
+        cnt += (io ? 1u : 0u) + (in ? 1u : 0u);
+        if (KIND == POT_HRSW) well += (int)in - (int)io;
+        else sum += (double)term(o, n, io, in);
+        more = go && (io || in);
+        ++k;
+    }
+    terms += go ? cnt : 0u;
+    return KIND == POT_HRSW ? -q.p1 * (double)well : sum;
+}
+
 // One displacement trial of particle i (block position t of a block of
 // length size, LDS address my) by md.  Same decisions as orc_trial_with: wall
 // test, hard core against the nearest partners (FP64), then the partner sums
@@ -684,29 +765,7 @@ __device__ __forceinline__ bool trial_lds(const LdsChain &c, const Pot &q, doubl
             const double bf = exp(-dE * beta);
             return go && (dE <= 0.0 || bf > u);
         }
-        double sS = 0.0;  // the side's FP32 pair terms summed in FP64
-        int wS = 0;  // hard rod + square well: the well count, as the one-lane walk
-        uint32_t k = 1;
-        if (__any(live)) {
-#pragma unroll 1
-        do {
-            const uint32_t jl = my - k - (k > t ? gapL : 0), jr = my + k + (t + k >= size ? gapR : 0);
-            const double xj = X[left ? jl : jr];
-            const double o = left ? xi - xj : xj - xi, nn = left ? xn - xj : xj - xn;
-            const bool io = inside64<KIND>(q, o), inn = inside64<KIND>(q, nn);
-            const bool in = live && walk_in<KIND>(q, o, nn, io, inn);
-            if (KIND == POT_HRSW) {
-                wS += in ? (int)inn - (int)io : 0;
-            } else {
-                // terms of partners off the walk are zero: exact no-op adds
-                sS += (double)(phi32<KIND>(q, (float)nn, in && inn) - phi32<KIND>(q, (float)o, in && io));
-            }
-            terms += n_walked<KIND>(in, io, inn);
-            live = in && k < kS;
-            ++k;
-        } while (__any(live));
-        }
-        const double mine = KIND == POT_HRSW ? -q.p1 * (double)wS : sS;
+        const double mine = walk_side32<KIND>(X, q, c.w, go, left, t, size, my, gapL, gapR, xi, xn, terms);
         dE = mine + __shfl_xor(mine, 1);
         const float bf = fexp(-betaf * (float)dE);
         return go && (dE <= 0.0 || (double)bf > u);
@@ -829,9 +888,22 @@ __device__ __forceinline__ bool trial_lds(const LdsChain &c, const Pot &q, doubl
     return go && (dE <= 0.0 || (double)bf > u);
 }
 
+// Where a block's box-length sums are cut in two: sums over the block
+// positions [0, h) and [h, size) are formed apart and added, so that two lanes
+// can share a block (the split kernel) and one lane gives the same bits.
+// Short blocks are not cut: the second walk would cost more than half of one
+// (the 20 sigma Yukawa chains, which the cut is for, have blocks of at least 41).
+constexpr uint32_t HALF_MIN = 40;
+
+__device__ __forceinline__ uint32_t half_of(uint32_t size)
+{
+    return size >= HALF_MIN ? (size + 1) / 2 : size;
+}
+
 // Box-length trial (fav, src/jmmMCState.cpp:2161-2293), one lane's share
-// over the pairs (i, i+k) whose left member is in the lane's block, in the
-// order t = 0.., k = 1.. : the energy change of scaling the configuration by
+// over the pairs (i, i+k) whose left member is at the block positions [t0, t1)
+// of the lane's block, in the
+// order t = t0.., k = 1.. : the energy change of scaling the configuration by
 // vp.sc pair by pair, FP64 form phi64(s d) - phi64(d), FP32 form box_term32
 // (one reciprocal per LJ pair through the scaling identity) summed in FP64;
 // each particle's walk ends at its first partner beyond
@@ -856,21 +928,22 @@ __device__ __forceinline__ bool trial_lds(const LdsChain &c, const Pot &q, doubl
 // pairwise sum gives.  W2: two partners of
 // a particle per iteration (for the common walk of one partner inside and
 // the next beyond the cutoff, one iteration per particle), same terms in
-// the same order.
+// the same order (four for the long windows of split chains: 4 % more
+// instructions, the walk's bookkeeping grew with them, and no time saved).
 template <typename Real, int KIND, bool W2 = false, typename Wrap>
 __device__ __forceinline__ double vol_lane(const LdsChain &c, const Pot &q, double gmin,
                                            const VolProp &vp, bool on, uint32_t start,
-                                           uint32_t size, uint32_t a0, uint32_t gapR, bool last,
-                                           Wrap wrap, uint32_t &bad, double &u0)
+                                           uint32_t size, uint32_t t0, uint32_t t1, uint32_t a0,
+                                           uint32_t gapR, bool last, Wrap wrap, uint32_t &bad, double &u0)
 {
     constexpr bool WELL = sizeof(Real) == 4 && KIND == POT_HRSW;
     const double *X = c.R;
     double part = 0.0;  // FP64 terms, or the FP32 form's FP32 terms summed in FP64
     int wc = 0;  // hard rod + square well, FP32: scaled pairs inside the well
     u0 = 0.0;    // FP32 form: the pairs' FP32 energy at the unscaled separations
-    bool run = on && size > 0;
-    uint32_t t = 0, k = 1;
-    double xi = X[run ? a0 : 0u];
+    bool run = on && t0 < t1;
+    uint32_t t = t0, k = 1;
+    double xi = X[run ? a0 + t0 : 0u];
     double xis = xi * vp.sc;
     double x1 = 0.0, x1s = 0.0;
     if (W2) {
@@ -924,7 +997,7 @@ __device__ __forceinline__ double vol_lane(const LdsChain &c, const Pot &q, doub
         // inside and more partners remain
         const bool nextp = !(add2 && k + 1 < kR);
         const uint32_t tn = nextp ? t + 1 : t;
-        run = run && !isbad && tn < size;
+        run = run && !isbad && tn < t1;
         xi = nextp ? x1 : xi;
         xis = nextp ? x1s : xis;
         k = nextp ? 1u : k + 2;
@@ -964,7 +1037,7 @@ __device__ __forceinline__ double vol_lane(const LdsChain &c, const Pot &q, doub
         // stepping t; their reads are redirected and their terms dropped)
         const bool nextp = !valid || stop || k == kR;
         const uint32_t tn = nextp ? t + 1 : t;
-        run = run && !isbad && tn < size;
+        run = run && !isbad && tn < t1;
         xi = nextp ? x1 : xi;
         xis = nextp ? x1s : xis;
         k = nextp ? 1u : k + 1;
@@ -1125,10 +1198,20 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
             vp = vol_propose(ch, L, sweep);
             auto wrap = [&](uint32_t m) { return c.R[c.wg + m]; };
             const bool last = c.per && r + 1 == c.B, von = vp.valid && act;
-            vpart = one ? vol_lane<Real, KIND, false>(c, q, gmin, vp, von, start, size, a0, gapR, last, wrap, bad,
-                                                      upart)
-                        : vol_lane<Real, KIND, sizeof(Real) == 4>(c, q, gmin, vp, von, start, size, a0, gapR, last,
-                                                                  wrap, bad, upart);
+            // long blocks in two halves (half_of; a bundle's longest decides)
+            const int parts = bd.smax >= HALF_MIN ? 2 : 1;
+            uint32_t t0 = 0, t1 = half_of(size);
+#pragma unroll 1
+            for (int part = 0; part < parts; ++part) {
+                double u = 0.0;
+                vpart += one ? vol_lane<Real, KIND, false>(c, q, gmin, vp, von, start, size, t0, t1, a0, gapR, last,
+                                                           wrap, bad, u)
+                             : vol_lane<Real, KIND, sizeof(Real) == 4>(c, q, gmin, vp, von, start, size, t0, t1, a0,
+                                                                       gapR, last, wrap, bad, u);
+                upart += u;
+                t0 = t1;
+                t1 = size;
+            }
         }
         {
             double v[3] = {dUs, vpart, upart};
@@ -1336,7 +1419,8 @@ __device__ __forceinline__ uint64_t seg_pidx(uint32_t j, uint32_t par, uint32_t 
 // block's state): they share each displacement trial, one walking the left
 // partners and one the right (trial_lds with PAIR), which halves the walk a
 // lane does and doubles the waves per CU when LDS limits the workgroups.
-// Everything else (loads, stores, the box-length and recompute sums) is the
+// The box-length sums of a block are cut in two halves (half_of), one lane
+// each.  Everything else (loads, stores, the recompute sums) is the
 // even lane's, and the sums are combined per 64 blocks as with one lane per
 // block, so LPB changes no result bit.  Sync points, the same in every
 // segment of a chain: the initial publication (neighbours); phases
@@ -1496,6 +1580,11 @@ __device__ __forceinline__ void run_segment(const SegArgs &g, const DevSeg &sg, 
         __syncthreads();
     };
 
+    // no partner beyond a wall: NaN is inside no cutoff (walk_side32)
+    for (uint32_t m = tid; m < wg; m += TW) {
+        if (!hasLn) c.R[m] = __longlong_as_double(0x7ff8000000000000ll);
+        if (!hasRn) c.R[wg + Bs * Sp + m] = __longlong_as_double(0x7ff8000000000000ll);
+    }
     publish_all();
     sync_nb();
     refresh();
@@ -1562,10 +1651,26 @@ __device__ __forceinline__ void run_segment(const SegArgs &g, const DevSeg &sg, 
         double vpart = 0.0, upart = 0.0;
         if (npt) {
             vp = vol_propose(ch, L, sweep);
-            vpart = vol_lane<Real, KIND, sizeof(Real) == 4>(
-                c, q, gmin, vp, vp.valid && act && own, start, size, a0, gapR,
-                per && r + 1 == Bs && s + 1 == S,
-                [&](uint32_t m) { return seg_load(&g.pub_head[(uint64_t)sg.first * W + m]); }, bad, upart);
+            const bool last = per && r + 1 == Bs && s + 1 == S, von = vp.valid && act;
+            auto wrap = [&](uint32_t m) { return seg_load(&g.pub_head[(uint64_t)sg.first * W + m]); };
+            const uint32_t h = half_of(size);
+            uint32_t t0 = own ? 0u : h, t1 = own ? h : size;
+            const bool two = LPB == 1 && __any(h < size);
+#pragma unroll 1
+            for (int part = 0; part < (two ? 2 : 1); ++part) {
+                double u = 0.0;
+                vpart += vol_lane<Real, KIND, sizeof(Real) == 4>(c, q, gmin, vp, von, start, size, t0, t1, a0, gapR,
+                                                                 last, wrap, bad, u);
+                upart += u;
+                t0 = t1;
+                t1 = size;
+            }
+            if (LPB == 2) {
+                // the two lanes' halves, on the lane that owns the block
+                const double v2 = __shfl_xor(vpart, 1), u2 = __shfl_xor(upart, 1);
+                vpart = own ? vpart + v2 : 0.0;
+                upart = own ? upart + u2 : 0.0;
+            }
         }
         const uint32_t par = (uint32_t)(sweep & 1u);
         {
@@ -1598,8 +1703,8 @@ __device__ __forceinline__ void run_segment(const SegArgs &g, const DevSeg &sg, 
             ++n_vt;
             const double dUv = (sizeof(Real) == 4 && KIND == POT_HRSW) ? tot[1] - U : tot[1];
             if (vp.valid && tot[3] == 0.0 && vol_accept(dUv, vp.dL, vp.lns, P, beta, vp.jac, vp.u)) {
-                if (own)
-                    for (uint32_t t = 0; t < size; ++t) c.R[a0 + t] = c.R[a0 + t] * vp.sc;
+                // the blocks' image as one array (its pads hold nothing)
+                for (uint32_t m = tid; m < Bs * Sp; m += TW) c.R[wg + m] = c.R[wg + m] * vp.sc;
                 L = vp.Lp;
                 U = U + dUv;
                 accv = 1;
