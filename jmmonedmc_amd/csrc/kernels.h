@@ -168,7 +168,8 @@ struct SampleRec {
 };
 static_assert(sizeof(SampleRec) == 24, "SampleRec must match jmm_sample");
 hipError_t launch_pack_samples(const double *sU, const double *sL, const uint2 *sA, const uint32_t *ext,
-                               uint32_t n_chains, uint32_t n_sweeps, SampleRec *out, hipStream_t s);
+                               uint32_t n_chains, uint32_t n_sweeps, SampleRec *out, Ctrl *ctrl, uint32_t n_ctrl,
+                               hipStream_t s);
 // Virial rows to the caller's layout: out[(ext[k] * n_sweeps + s) * 2 + {0, 1}]
 // = (W, HV) of sweep s.
 hipError_t launch_pack_virials(const double *sW, const double *sH, const uint32_t *ext, uint32_t n_chains,

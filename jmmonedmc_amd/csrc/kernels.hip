@@ -2162,11 +2162,14 @@ __global__ void __launch_bounds__(64) k_obs_sum(ObsArgs a)
 // Sample rows [sweep][chain] (internal chain order) to the caller's layout
 // [chain][sweep] (external order), through 32 x 32 tiles in LDS so that the
 // reads (along chains) and the writes (along sweeps) are both contiguous.
-// Grid-stride over tiles.
+// Grid-stride over tiles.  Also empties the sample buffer (n_ctrl <= 256
+// queues).
 __global__ void __launch_bounds__(256) k_pack_samples(const double *sU, const double *sL, const uint2 *sA,
                                                       const uint32_t *ext, uint32_t nc, uint32_t ns,
-                                                      SampleRec *out)
+                                                      SampleRec *out, Ctrl *ctrl, uint32_t n_ctrl)
 {
+    // the read empties the sample buffer: the queues' rows start over
+    if (blockIdx.x == 0 && threadIdx.x < n_ctrl) ctrl[threadIdx.x].next_off = 0;
     __shared__ double tU[32][33], tL[32][33];
     __shared__ uint2 tA[32][33];
     const uint32_t tx = threadIdx.x & 31u, ty = threadIdx.x >> 5;
@@ -2402,12 +2405,14 @@ hipError_t launch_pack_virials(const double *sW, const double *sH, const uint32_
 }
 
 hipError_t launch_pack_samples(const double *sU, const double *sL, const uint2 *sA, const uint32_t *ext,
-                               uint32_t n_chains, uint32_t n_sweeps, SampleRec *out, hipStream_t s)
+                               uint32_t n_chains, uint32_t n_sweeps, SampleRec *out, Ctrl *ctrl, uint32_t n_ctrl,
+                               hipStream_t s)
 {
     const uint64_t tiles = (uint64_t)((n_chains + 31u) / 32u) * ((n_sweeps + 31u) / 32u);
     const uint32_t grid = (uint32_t)std::min<uint64_t>(tiles, 1u << 16);
     if (!grid) return hipSuccess;
-    hipLaunchKernelGGL(k_pack_samples, dim3(grid), dim3(256), 0, s, sU, sL, sA, ext, n_chains, n_sweeps, out);
+    hipLaunchKernelGGL(k_pack_samples, dim3(grid), dim3(256), 0, s, sU, sL, sA, ext, n_chains, n_sweeps, out, ctrl,
+                       n_ctrl);
     return hipGetLastError();
 }
 
