@@ -109,7 +109,10 @@ typedef struct jmm_engine_opts {
     uint32_t sample_virial;   /* 1: after every sweep each chain's virial W = sum -d phi'(d)
                                  and hypervirial sum -d W'(d) are computed (FP64) and kept
                                  with the samples (jmm_read_samples_virial) */
-    uint32_t reserved;
+    uint32_t block_lanes;     /* batched forms, chains that are not split: 0 = chosen by the
+                                 number of chains, 1 = one lane per block of particles, 2 or
+                                 more = several (a workgroup per chain) where every chain's
+                                 window allows it; results are the same bits either way */
 } jmm_engine_opts;
 
 /* One per chain per sweep (the per-sweep form of the reference's per-trial

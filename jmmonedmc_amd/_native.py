@@ -45,7 +45,7 @@ class EngineOpts(C.Structure):
         ("form", C.c_int32), ("device", C.c_int32), ("sample_capacity", C.c_uint32),
         ("block_sweeps", C.c_uint32), ("wg_threads", C.c_uint32), ("use_graph", C.c_uint32),
         ("log_accepts", C.c_uint32), ("lds_budget", C.c_uint32), ("seg_lds", C.c_uint32),
-        ("seg_lanes", C.c_uint32), ("sample_virial", C.c_uint32), ("reserved", C.c_uint32),
+        ("seg_lanes", C.c_uint32), ("sample_virial", C.c_uint32), ("block_lanes", C.c_uint32),
     ]
 
 

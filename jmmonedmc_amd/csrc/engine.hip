@@ -262,13 +262,36 @@ int dalloc(T **p, size_t n)
 
 struct Group {
     int gx = 0;
-    int kind = 0;
+    int coop = 0;             // cooperative form: n_items chains in d_list
+    uint32_t threads = 0;     // lanes per workgroup (cooperative form)
     uint32_t n_items = 0;     // bundles (batched) or chains (plain)
     uint32_t grid = 0;
     size_t lds = 0;
     DevBundle *d_bundles = nullptr;
     uint32_t *d_list = nullptr;
 };
+
+// Most waves per CU (of its 32) at which an engine's chains run one per
+// workgroup with several lanes per block: beyond, the extra lanes' work costs
+// more than the latency they save.  us per sweep, one lane -> several, LJ NPT
+// FP32: 1024 chains of 64 (8 waves per CU) 17.9 -> 10.6, 2048 (16) 17.9 -> 26.9;
+// 256 of 250 (8) 17.5 -> 11.2, 512 (16) 17.7 -> 22.0.
+constexpr uint64_t COOP_WAVES = 8;
+
+// Phases of a sweep times the partners of a trial, by which chains end.
+static uint64_t chain_cost(const DevChain &c) { return (uint64_t)c.smax * (c.w + 2); }
+
+// Whether a chain runs faster with several lanes per block when it has the CU
+// to itself: with more than one partner a side and at least 4 lanes per block
+// (up to 128 blocks), or with two partners a side (2 lanes per block take them
+// at once).  us per sweep, FP32 / FP64: LJ chains (6 partners) of 64 17.2 -> 8.4
+// / 22.6 -> 9.1, of 1000 (128 blocks) 17.5 -> 14.5 / 23.2 -> 15.1, of 4000 (256
+// blocks) 31.0 -> 32.9 / 42.4 -> 41.5; hard rods with a well (1 partner) of 64
+// 4.7 -> 5.4, of 1000 6.9 -> 7.6.
+static bool coop_gains(const DevChain &c)
+{
+    return c.w >= 2 && (c.B <= 128 || c.w == 2);
+}
 
 struct jmm_engine {
     int n = 0, form = 0, device = 0, T = 256;
@@ -384,6 +407,8 @@ int launch_block(jmm_engine *e, uint32_t m)
         a.cap = e->cap;
         if (e->form == JMM_FORM_PLAIN_FP64) {
             HIPCHK(launch_plain(a, G.gx, G.grid, G.lds, e->stream));
+        } else if (G.coop) {
+            HIPCHK(launch_coop(a, e->form == JMM_FORM_BATCHED_FP32, G.grid, G.threads, G.lds, e->stream));
         } else {
             HIPCHK(launch_batched(a, e->form == JMM_FORM_BATCHED_FP32, e->T, G.gx, G.grid, G.lds,
                                   e->stream));
@@ -666,6 +691,23 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
     for (int c = 0; c < n_chains; ++c)
         if (!segS[c]) maxB = std::max(maxB, ch[c].B);
 
+    // Engines with too few chains to fill the GPU give each a workgroup with
+    // several lanes per block (k_sweep_coop), where every chain that is not
+    // split is short-ranged enough for it, the longest gains by it (coop_gains;
+    // the others end before it) and all of them are resident at COOP_WAVES
+    // waves per CU.
+    bool coop = e->form != JMM_FORM_PLAIN_FP64 && o.block_lanes != 1;
+    uint64_t coop_waves = 0;
+    int longest = -1;
+    for (int c = 0; c < n_chains && coop; ++c) {
+        if (segS[c]) continue;
+        if (ch[c].w > COOP_W || ch[c].B > COOP_B || coop_lds(ch[c]) > (size_t)lds_max - 1024) coop = false;
+        coop_waves += coop_threads(ch[c]) / 64;
+        if (longest < 0 || chain_cost(ch[c]) > chain_cost(ch[longest])) longest = c;
+    }
+    coop = coop && longest >= 0 &&
+           (o.block_lanes > 1 || (coop_gains(ch[longest]) && coop_waves <= (uint64_t)n_cu * COOP_WAVES));
+
     // internal chain order and bundles (segmented chains last)
     std::vector<DevBundle> bundles[2];
     std::vector<DevSlot> slots;
@@ -680,7 +722,16 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
         if (maxB > 1024) return bail(fail(JMM_EINVAL, "jmm_create: more than 1024 blocks in a chain"));
         size_t budget = o.lds_budget ? o.lds_budget : 65536;
         budget = std::min<size_t>(budget, (size_t)lds_max);
-        PackOut p = pack(e->specs, ch, e->T, budget / 8, (size_t)lds_max / 8 - 64, segS);
+        PackOut p;
+        if (coop) {
+            // the longest first: they end last
+            for (int c = 0; c < n_chains; ++c)
+                if (!segS[c]) p.order.push_back((uint32_t)c);
+            std::stable_sort(p.order.begin(), p.order.end(),
+                             [&](uint32_t x, uint32_t y) { return chain_cost(ch[x]) > chain_cost(ch[y]); });
+        } else {
+            p = pack(e->specs, ch, e->T, budget / 8, (size_t)lds_max / 8 - 64, segS);
+        }
         order = p.order;
         for (int c = 0; c < n_chains; ++c)
             if (segS[c]) order.push_back((uint32_t)c);
@@ -707,7 +758,8 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
             l.mode = JMM_MODE_HBM;
         } else {
             l.mode = JMM_MODE_LDS;
-            l.lds_bytes = sizeof(double) * (uint64_t)ch[c].lds_len;
+            l.lds_bytes = coop ? (uint64_t)coop_lds(ch[c]) : sizeof(double) * (uint64_t)ch[c].lds_len;
+            if (coop) l.lanes = coop_lanes(ch[c].B);
         }
     }
     e->ext_of_int = order;
@@ -784,6 +836,23 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
             CREATE_CHK(hipMemcpy(Gr.d_list, lists[g].data(), sizeof(uint32_t) * Gr.n_items, hipMemcpyHostToDevice));
         }
     } else {
+        if (coop) {
+            Group G;
+            G.coop = 1;
+            std::vector<uint32_t> list;
+            for (int k = 0; k < n_chains; ++k) {
+                if (segS[order[k]]) continue;
+                list.push_back((uint32_t)k);
+                G.threads = std::max(G.threads, coop_threads(e->hch[k]));
+                G.lds = std::max(G.lds, coop_lds(e->hch[k]));
+            }
+            G.n_items = G.grid = (uint32_t)list.size();
+            if (int rc = set_lds_attr(coop_kernel(e->form == JMM_FORM_BATCHED_FP32), G.lds)) return bail(rc);
+            e->grp.push_back(G);
+            Group &Gc = e->grp.back();
+            if (int rc = dalloc(&Gc.d_list, Gc.n_items)) return bail(rc);
+            CREATE_CHK(hipMemcpy(Gc.d_list, list.data(), sizeof(uint32_t) * Gc.n_items, hipMemcpyHostToDevice));
+        }
         if (int rc = dalloc(&e->d_slots, slots.size())) return bail(rc);
         CREATE_CHK(hipMemcpy(e->d_slots, slots.data(), sizeof(DevSlot) * slots.size(), hipMemcpyHostToDevice));
         for (int g = 0; g < 2; ++g) {

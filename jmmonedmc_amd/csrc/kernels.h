@@ -156,6 +156,16 @@ hipError_t launch_begin(Ctrl *c, uint32_t n, hipStream_t s);
 const void *batched_kernel(int fp32, int T, int gx);
 hipError_t launch_batched(const SweepArgs &a, int fp32, int T, int gx, uint32_t grid, size_t lds,
                           hipStream_t s);
+// Cooperative form: one chain per workgroup of at most COOP_T lanes (512: two
+// waves per SIMD, so 256 registers; 1024 lanes with 128 spilled), 16, 4 or 2
+// lanes per block; chains with at most COOP_W partners per side and COOP_B
+// blocks.
+constexpr uint32_t COOP_W = 8, COOP_B = 256, COOP_T = 512;
+__host__ __device__ inline uint32_t coop_lanes(uint32_t B) { return B <= 32 ? 16u : B <= 128 ? 4u : 2u; }
+size_t coop_lds(const DevChain &c);
+uint32_t coop_threads(const DevChain &c);
+const void *coop_kernel(int fp32);
+hipError_t launch_coop(const SweepArgs &a, int fp32, uint32_t grid, uint32_t threads, size_t lds, hipStream_t s);
 const void *plain_kernel(int gx);
 hipError_t launch_plain(const SweepArgs &a, int gx, uint32_t grid, size_t lds, hipStream_t s);
 hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads,

@@ -246,6 +246,7 @@ struct VolProp {
 
 // Out of line: its FP64 log/exp/division temporaries would otherwise raise
 // the register count of the whole sweep loop.
+template <typename Real>
 __device__ __noinline__ VolProp vol_propose(const DevChain &ch, double L, uint64_t sweep)
 {
     uint32_t r[4];
@@ -269,10 +270,13 @@ __device__ __noinline__ VolProp vol_propose(const DevChain &ch, double L, uint64
         v.dL = v.Lp - L;
     }
     v.valid = v.Lp > 0.0 && (!(ch.flags & F_PERIODIC) || v.Lp > ch.Lmin);
-    // s^-12 - 1 and s^-6 - 1 from expm1 of ln s: no cancellation
-    const double a6 = ch.pot.e4 * ch.pot.sig6;
-    v.bk.c12 = (float)(a6 * ch.pot.sig6 * expm1(-12.0 * v.lns));
-    v.bk.c6 = (float)(a6 * expm1(-6.0 * v.lns));
+    v.bk.c12 = v.bk.c6 = 0.0f;
+    if (sizeof(Real) == 4) {
+        // s^-12 - 1 and s^-6 - 1 from expm1 of ln s: no cancellation
+        const double a6 = ch.pot.e4 * ch.pot.sig6;
+        v.bk.c12 = (float)(a6 * ch.pot.sig6 * expm1(-12.0 * v.lns));
+        v.bk.c6 = (float)(a6 * expm1(-6.0 * v.lns));
+    }
     return v;
 }
 
@@ -459,7 +463,7 @@ __device__ __forceinline__ void run_bundle_gx(const SweepArgs &a, const DevBundl
         uint32_t bad = 0;
         double vpart = 0.0, upart = 0.0;
         if (npt) {
-            vp = vol_propose(ch, L, sweep);
+            vp = vol_propose<Real>(ch, L, sweep);
             if (vp.valid && act)
                 vpart = scaled_delta<Real, KIND>(q, vp.bk, gmin, X, N, per, L, vp.Lp, vp.sc, w, start,
                                                  start + size, 1, bad, upart);
@@ -567,27 +571,16 @@ struct LdsChain {
     bool per;
 };
 
-__device__ __forceinline__ uint32_t lds_addr(const LdsChain &c, uint32_t i)
-{
-    const uint32_t big = c.rem * (c.qb + 1);
-    uint32_t b, t;
-    if (i < big) {
-        b = i / (c.qb + 1);
-        t = i - b * (c.qb + 1);
-    } else {
-        b = c.rem + (i - big) / c.qb;
-        t = i - (b * c.qb + c.rem);
-    }
-    return c.wg + b * c.Sp + t;
-}
-
-// Images of the first and last wg particles; lanes r = 0..B-1 share the work.
-__device__ __forceinline__ void fill_ghosts(const LdsChain &c, uint32_t r, double L)
+// Images of the first and last wg particles, lanes r = 0 .. n - 1 sharing the
+// work.  They lie in the first and the last block (a block holds at least
+// M_min >= wg particles, or all of them).
+__device__ __forceinline__ void fill_ghosts(const LdsChain &c, uint32_t r, uint32_t n, double L)
 {
     if (!c.per) return;
-    for (uint32_t m = r; m < c.wg && m < c.N; m += c.B) {
-        c.R[c.wg + c.B * c.Sp + m] = c.R[lds_addr(c, m)] + L;
-        c.R[m] = c.R[lds_addr(c, c.N - c.wg + m)] - L;
+    const uint32_t tail = c.wg + (c.B - 1) * c.Sp + (c.qb + (c.B - 1 < c.rem ? 1u : 0u)) - c.wg;
+    for (uint32_t m = r; m < c.wg; m += n) {
+        c.R[c.wg + c.B * c.Sp + m] = c.R[c.wg + m] + L;
+        c.R[m] = c.R[tail + m] - L;
     }
 }
 
@@ -1130,7 +1123,7 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
     double L = st.L, U = st.U, mdrift = st.max_drift;
     uint64_t sweep = st.sweep;
     __syncthreads();
-    if (act) fill_ghosts(c, r, L);
+    if (act) fill_ghosts(c, r, c.B, L);
     __syncthreads();
 
     uint32_t n_tr = 0, n_wall = 0, n_core = 0, n_terms = 0;
@@ -1195,7 +1188,7 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
         uint32_t bad = 0;
         double vpart = 0.0, upart = 0.0;
         if (npt) {
-            vp = vol_propose(ch, L, sweep);
+            vp = vol_propose<Real>(ch, L, sweep);
             auto wrap = [&](uint32_t m) { return c.R[c.wg + m]; };
             const bool last = c.per && r + 1 == c.B, von = vp.valid && act;
             // long blocks in two halves (half_of; a bundle's longest decides)
@@ -1243,7 +1236,7 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
             __syncthreads();
             // only the chain's own lanes: idle lanes of the workgroup carry no
             // energy partials and so no valid decision
-            if (accv && act) fill_ghosts(c, r, L);
+            if (accv && act) fill_ghosts(c, r, c.B, L);
             __syncthreads();
         }
 
@@ -1356,6 +1349,666 @@ k_sweep_batched(SweepArgs a)
             }
         }
         __syncthreads();
+    }
+}
+
+// --------------------------------------------------------- cooperative form
+
+// Data-parallel control that gives every lane of a group of G lanes lane I's
+// value: row_newbcast:I, quad_perm:[I,I,I,I], quad_perm:[I,I,2+I,2+I].
+template <int G, int I>
+constexpr int lane_ctrl()
+{
+    return G == 16 ? 0x150 + I : G == 4 ? I * 0x55 : 0xA0 + I * 0x55;
+}
+
+// The value of lane I of the caller's group of G lanes (16: a row; 4: a
+// quad; 2), through the data-parallel primitives: no LDS round trip.
+template <int G, int I>
+__device__ __forceinline__ double from_lane(double v)
+{
+    constexpr int ctrl = lane_ctrl<G, I>();
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+template <int G, int I>
+__device__ __forceinline__ int from_lane_i(int v)
+{
+    return __builtin_amdgcn_mov_dpp(v, lane_ctrl<G, I>(), 0xf, 0xf, true);
+}
+
+// exp out of line: its constants would otherwise sit in registers through the
+// phases, where it is almost never needed.
+__device__ __noinline__ double exp_apart(double x) { return exp(x); }
+
+// phi64 of a separation whose cutoff test has been made, without branches
+// (hard cores are handled before any pair is evaluated).
+template <int KIND>
+__device__ __forceinline__ double phi64_in(const Pot &q, double d, bool in)
+{
+    double v;
+    if (KIND == POT_LJ) {
+        const double d3 = d * d * d;
+        const double i6 = (1.0 / (d3 * d3)) * q.sig6;
+        const double i12 = i6 * i6;
+        v = (q.e4 * i12 - q.e4 * i6) - q.shift;
+    } else if (KIND == POT_HARMONIC) {
+        const double m = d - 1.0;
+        v = d <= 0.0 ? 10e10 : m * m;
+    } else if (KIND == POT_HRSW) {
+        v = -q.p1;
+    } else {
+        v = (q.p0 * (exp(-q.p1 * d) / d)) - q.shift;
+    }
+    return in ? v : 0.0;
+}
+
+// acc plus the group's lanes I0, I0 + 1, ... I1 - 1, each lane's KP terms in
+// turn.
+template <int G, int I0, int I1, uint32_t KP>
+__device__ __forceinline__ double add_lanes(double acc, const double (&v)[KP])
+{
+    if constexpr (I0 < I1) {
+#pragma unroll
+        for (uint32_t u = 0; u < KP; ++u) acc += from_lane<G, I0>(v[u]);
+        return add_lanes<G, I0 + 1, I1, KP>(acc, v);
+    } else {
+        return acc;
+    }
+}
+
+// One side's ordered sum of a trial's terms (the group's lanes I0 .. I0 +
+// G/2 - 1), the far lanes only where some trial of the wave reaches them:
+// some lane's h of at least 1, 2, 4 holds a partner inside the cutoff
+// (uniform); the terms left out are zeros.
+template <int G, int I0, uint32_t KP>
+__device__ __forceinline__ double add_side(double acc, const double (&v)[KP], bool far1, bool far2, bool far4)
+{
+    constexpr int H = G / 2;
+    acc = add_lanes<G, I0, I0 + 1, KP>(acc, v);
+    if constexpr (H > 1) {
+        if (far1) {
+            acc = add_lanes<G, I0 + 1, I0 + 2, KP>(acc, v);
+            if constexpr (H > 2) {
+                if (far2) {
+                    acc = add_lanes<G, I0 + 2, I0 + 4, KP>(acc, v);
+                    if (far4) acc = add_lanes<G, I0 + 4, I0 + H, KP>(acc, v);
+                }
+            }
+        }
+    }
+    return acc;
+}
+
+// What the waves of a workgroup share: the sweep's box-length proposal, its
+// integer totals (two slots, by sweep parity: one is cleared while the other
+// is read) and the 64-block sums, and the launch's counters.
+struct CoopScratch {
+    VolProp vp;
+    double grp[COOP_B / 64][3];
+    uint32_t acc[2], bad[2];
+    uint32_t wall, core, terms;
+};
+
+// Sum of a block's pair terms in the order of the one-lane walks (particle by
+// particle, each particle's partners outwards): the G lanes of the block take
+// a particle each, put their terms into LDS and all add them in sequence, so
+// every lane holds the one-lane sum bit for bit.  pair(k, t, xi, xj, v) sets
+// a pair's NF terms and returns whether the particle's walk goes on; a partner
+// after the last has zero terms, whose addition is exact.
+template <int G, int NF, typename Pair>
+__device__ __forceinline__ void block_sum(const LdsChain &c, uint32_t start, uint32_t size, uint32_t t0, uint32_t t1,
+                                          uint32_t a0, uint32_t gapR, uint32_t g, double *terms, double (&acc)[NF],
+                                          Pair pair)
+{
+    for (uint32_t tb = t0; __any(tb < t1); tb += G) {
+        const uint32_t t = tb + g;
+        bool run = t < t1;
+        const double xi = c.R[run ? a0 + t : 0u];
+        const uint32_t kR = c.per ? c.w : min(c.w, c.N - 1 - (start + t));
+        double v[NF][COOP_W];
+        uint32_t kmax = 0;
+        // two partners at a time: their reads and pair energies overlap
+#pragma unroll
+        for (uint32_t k = 1; k <= COOP_W; k += 2) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) v[f][k - 1] = v[f][k] = 0.0;
+            if (k <= c.w) {
+                run = run & (k <= kR);
+                if (__any(run)) {
+                    const bool run2 = run & (k + 1 <= kR);
+                    const double xj = c.R[run ? a0 + t + k + (t + k >= size ? gapR : 0u) : 0u];
+                    const double xj2 = c.R[run2 ? a0 + t + k + 1 + (t + k + 1 >= size ? gapR : 0u) : 0u];
+                    double q[NF], q2[NF];
+                    const bool on = pair(k, t, xi, xj, run, q) & run;
+                    const bool on2 = pair(k + 1, t, xi, xj2, run2, q2) & run2 & on;
+#pragma unroll
+                    for (int f = 0; f < NF; ++f) {
+                        v[f][k - 1] = on ? q[f] : 0.0;
+                        v[f][k] = on2 ? q2[f] : 0.0;
+                    }
+                    kmax = min(k + 1, c.w);
+                    run = on2;
+                }
+            }
+        }
+        // the group's terms, lane-major; a wave's own lanes only: LDS keeps a
+        // wave's order, the fences keep the compiler's
+        const uint32_t M = G * kmax;
+        double *mine = terms + (threadIdx.x / G) * (G * c.w * NF);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (uint32_t k = 0; k < COOP_W; ++k)
+            if (k < kmax)
+#pragma unroll
+                for (int f = 0; f < NF; ++f) mine[f * M + g * kmax + k] = v[f][k];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        constexpr int E = G < 4 ? G : 4;
+        for (uint32_t m = 0; m < M; m += E) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                double e[E];
+#pragma unroll
+                for (int u = 0; u < E; ++u) e[u] = mine[f * M + m + u];
+#pragma unroll
+                for (int u = 0; u < E; ++u) acc[f] += e[u];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// v plus the value of the lane with one bit of its index flipped, for values
+// that are already equal within the smaller halves (so a mirrored lane of the
+// other half does): inside a row without an LDS round trip.
+template <int OFF, int ND>
+__device__ __forceinline__ void add_xor(double (&v)[ND])
+{
+#pragma unroll
+    for (int m = 0; m < ND; ++m) {
+        if constexpr (OFF >= 16) {
+            v[m] += __shfl_xor(v[m], OFF);
+        } else {
+            // quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror, row_mirror
+            constexpr int ctrl = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x140;
+            const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v[m]), ctrl, 0xf, 0xf, true);
+            const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v[m]), ctrl, 0xf, 0xf, true);
+            v[m] += __hiloint2double(hi, lo);
+        }
+    }
+}
+
+// Sums over the chain's blocks in the order of seg_allreduce (pairwise trees
+// over 64 blocks, then the trees in sequence), from per-block values in LDS:
+// one wave per 64 blocks, a block per lane; every lane of the workgroup
+// receives the same bits.  Contains a workgroup barrier.
+template <int ND>
+__device__ __forceinline__ void chain_sum(const double *blk, uint32_t B, CoopScratch &sc, double (&v)[ND])
+{
+    const uint32_t l = threadIdx.x & 63u, q = threadIdx.x >> 6, top = B < 64 ? B : 64u;
+    if (q * 64 < B) {
+        double p[ND];
+#pragma unroll
+        for (int m = 0; m < ND; ++m) p[m] = l < top ? blk[m * B + q * 64 + l] : 0.0;
+        if (top > 1) add_xor<1>(p);
+        if (top > 2) add_xor<2>(p);
+        if (top > 4) add_xor<4>(p);
+        if (top > 8) add_xor<8>(p);
+        if (top > 16) add_xor<16>(p);
+        if (top > 32) add_xor<32>(p);
+        if (l == 0)
+#pragma unroll
+            for (int m = 0; m < ND; ++m) sc.grp[q][m] = p[m];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < ND; ++m) {
+        double acc = sc.grp[0][m];
+        for (uint32_t k = 1; k * 64 < B; ++k) acc += sc.grp[k][m];
+        v[m] = acc;
+    }
+}
+
+// One chain per workgroup, G lanes per block, for engines with too few
+// chains to fill the GPU: a phase's time is then the latency of one trial,
+// and the batched kernel's lane walks its partners, its random numbers and
+// (box-length move, recompute, virial) its block's pairs one after another.
+// Here the partners of a trial are G/2 lanes a side at once, the random
+// numbers of the next 2 G block positions are drawn G lanes at once before
+// them (with ln u in the FP64 form, so that the Metropolis exponential is
+// evaluated only where |ln u + beta dE| < 1e-4: outside, the comparison of the
+// logarithms decides the same, |ln u| < 23 from the hardware's FP32 logarithm
+// being good to 1e-5), and the sums over a block's pairs take a
+// particle per lane.  Trials, random numbers and the order of every sum are
+// run_bundle_lds's, so a chain has the same bits in both.
+//
+// Bound by the latency of a phase: about 120 vector and 65 scalar
+// instructions of one wave (some 5 cycles each), two dependent LDS reads and a
+// barrier.  One LJ chain of 64, FP64: 0.56 us a phase where the batched
+// kernel takes 1.9 (100 sweeps and their read: 1494 -> 593 us); 64 chains of
+// 32 to 256, both potentials, FP32 NPT: 3154 -> 1158 us; one chain of 2000
+// with two partners a side, virials, FP64: 10 sweeps 294 -> 254 us.
+template <typename Real, int KIND, int G, uint32_t KP>
+__device__ __forceinline__ void run_coop(const SweepArgs &a, uint32_t ic, double *smem, CoopScratch &sc, uint32_t soff)
+{
+    constexpr uint32_t H = G / 2;  // lanes a side
+    constexpr bool WELL = sizeof(Real) == 4 && KIND == POT_HRSW;
+    constexpr uint32_t GM = (1u << G) - 1;
+    const uint32_t tid = threadIdx.x, T = blockDim.x, lane = tid & 63u;
+    const DevChain &ch = a.chains[ic];
+    const Pot q = ch.pot;
+    const double gmin = ch.gmin, max_step = ch.max_step, beta = ch.beta, P = ch.P;
+    const float betaf = ch.betaf;
+    const uint32_t key0 = (uint32_t)ch.seed, key1 = (uint32_t)(ch.seed >> 32);
+    const uint32_t chain_id = ch.chain_id, eci = ch.eci;
+    const uint64_t log_off = ch.log_off;
+    const bool npt = (ch.flags & F_NPT) != 0;
+    const uint32_t smax = ch.smax;
+
+    LdsChain c;
+    c.R = smem;
+    c.N = ch.N;
+    c.B = ch.B;
+    c.w = ch.w;
+    c.wg = ch.wg;
+    c.Sp = ch.Sp;
+    c.qb = ch.N / ch.B;
+    c.rem = ch.N % ch.B;
+    c.per = (ch.flags & F_PERIODIC) != 0;
+    double *blk = smem + ch.lds_len;   // [3][B]: per-block sums
+    double *work = blk + 3 * c.B;      // random numbers, or pair terms
+    double2 *rnd = (double2 *)(work + ((ch.lds_len + 3 * c.B) & 1u));
+    uint32_t *rndw = (uint32_t *)(rnd + (size_t)c.B * 2 * G);
+
+    const uint32_t b = tid / G, g = tid % G;
+    const bool act = b < c.B;
+    const uint32_t size = act ? c.qb + (b < c.rem ? 1u : 0u) : 0u;
+    const uint32_t start = act ? b * c.qb + (b < c.rem ? b : c.rem) : 0u;
+    const uint32_t a0 = c.wg + b * c.Sp;
+    const uint32_t gapR = c.Sp - size;
+    const uint32_t gapL = b == 0 ? 0u : c.Sp - (c.qb + (b - 1 < c.rem ? 1u : 0u));
+    const bool left = g < H;
+    const uint32_t h = left ? g : g - H;
+    const uint32_t gl = lane & ~(uint32_t)(G - 1);  // the group's first lane in its wave
+    const uint32_t dir = left ? ~0u : 1u, gap = left ? 0u - gapL : gapR;
+    // what the lane stores after a trial: the particle (lane 0), its image in
+    // the right (lane 1) or left (lane 2) ghosts; putb + t for the block
+    // positions t of [put0, put0 + putn)
+    uint32_t putb = a0, put0 = 0, putn = g == 0 ? size : 0u;
+    double puts = 0.0;
+    if (c.per && g == 1 && start < c.wg) {
+        putb = c.wg + c.B * c.Sp + start;
+        putn = c.wg - start;
+        puts = 1.0;
+    }
+    // (two lanes per block: chains of many blocks, the last not the first)
+    if (c.per && g == (G == 2 ? 1 : 2) && size && start + size + c.wg > c.N) {
+        put0 = start + c.wg < c.N ? c.N - c.wg - start : 0u;
+        putb = start + c.wg - c.N;  // modulo 2^32 below put0
+        putn = size - put0;
+        puts = -1.0;
+    }
+
+    const double *xg = a.x + ch.x_off;
+    for (uint32_t t = g; t < size; t += G) c.R[a0 + t] = xg[start + t];
+    const DevState st = a.states[ic];
+    double L = st.L, U = st.U, mdrift = st.max_drift;
+    uint64_t sweep = st.sweep;
+    if (tid == 0) {
+        sc.acc[0] = sc.acc[1] = sc.bad[0] = sc.bad[1] = 0;
+        sc.wall = sc.core = sc.terms = 0;
+    }
+    __syncthreads();
+    fill_ghosts(c, tid, T, L);
+    __syncthreads();
+
+    // rejections per block, pair terms per lane
+    uint32_t n_wall = 0, n_core = 0, n_terms = 0;
+    uint32_t acc_total = 0, n_vt = 0, n_av = 0, n_rc = 0;
+
+#pragma unroll 1
+    for (uint32_t sw = 0; sw < a.n_sweeps; ++sw, ++sweep) {
+        double dUs = 0.0;
+        uint32_t acc = 0;
+        const double putL = puts * L;
+        // the sweep's box-length proposal depends on L alone: the last wave
+        // (the shortest blocks) prepares it
+        if (npt && tid >= T - 64) {
+            const VolProp v = vol_propose<Real>(ch, L, sweep);
+            if (lane == 0) sc.vp = v;
+        }
+#pragma unroll 1
+        for (uint32_t t = 0; t < smax; ++t) {
+            const uint32_t tr = t & (2 * G - 1);
+            if (tr == 0) {
+                // random numbers of the block positions t .. t + 2 G - 1
+                const uint32_t j = t + 2 * g;
+                if (j < size) {
+                    uint32_t rr[4];
+                    philox4x32_10(start + j, (uint32_t)sweep, chain_id, 0u, key0, key1, rr);
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) {
+                        const double u = u32o(rr[2 * m + 1]);
+                        const uint32_t at = b * 2 * G + 2 * g + m;
+                        rnd[at] = make_double2(((u32o(rr[2 * m]) - 0.5) * 2.0) * max_step,
+                                               sizeof(Real) == 8 ? (double)__logf((float)u) : u);
+                        if (sizeof(Real) == 8) rndw[at] = rr[2 * m + 1];
+                    }
+                }
+                __syncthreads();
+            }
+            if (t < size) {
+                const uint32_t i = start + t, my = a0 + t;
+                const uint32_t ri = b * 2 * G + tr;
+                // partner k0 + h + 1 on the lane's side (clamped to the image)
+                const uint32_t side_n = c.per ? UINT32_MAX : left ? i : c.N - 1 - i;
+                const uint32_t own_n = left ? t : size - 1 - t;  // partners in the own block
+                auto partner = [&](uint32_t k) {
+                    const uint32_t kk = min(k, c.wg);
+                    return c.R[my + dir * kk + (kk > own_n ? gap : 0u)];
+                };
+                double xj[KP];
+#pragma unroll
+                for (uint32_t u = 0; u < KP; ++u) xj[u] = partner(h * KP + u + 1);
+                const double2 rn = rnd[ri];
+                const double xi = c.R[my];
+                const double xn = xi + rn.x;
+                const bool wall = !c.per && fabs(xn) > L / 2.0;
+                const double s0 = xn - xj[0], sn = left ? s0 : -s0;
+                // the nearest partners' hard-core test, on one lane a side
+                const int hit = (int)((h == 0) & (c.N >= 2) & (side_n >= 1) & (sn < gmin));
+                const bool core = (from_lane_i<G, 0>(hit) | from_lane_i<G, H>(hit)) != 0;
+                const bool go = !wall & !core;
+                n_wall += wall ? 1u : 0u;
+                n_core += !wall & core ? 1u : 0u;
+                double dEL = 0.0, dER = 0.0, side = 0.0;
+                int wL = 0, wR = 0;
+                uint32_t k0 = 0;
+                for (;;) {
+                    // all evaluated on every lane, side by side: a branch
+                    // each would run them one after the other
+                    double term[KP];
+                    uint64_t any = 0, last_in = 0;
+#pragma unroll
+                    for (uint32_t u = 0; u < KP; ++u) {
+                        const uint32_t k = k0 + h * KP + u + 1;
+                        const double o = fabs(xi - xj[u]), n = fabs(xn - xj[u]);
+                        const bool valid = go & (k <= c.w) & (k <= side_n);
+                        const bool io = valid & inside64<KIND>(q, o), in = valid & inside64<KIND>(q, n);
+                        n_terms += (io ? 1u : 0u) + (in ? 1u : 0u);
+                        const uint64_t bo = __ballot(io), bn = __ballot(in);
+                        last_in = bo | bn;
+                        any |= last_in;
+                        if (WELL) {
+                            const uint32_t mo = (uint32_t)(bo >> gl) & GM, mn = (uint32_t)(bn >> gl) & GM;
+                            constexpr uint32_t LM = (1u << H) - 1;
+                            wL += (int)__popc(mn & LM) - (int)__popc(mo & LM);
+                            wR += (int)__popc(mn & ~LM) - (int)__popc(mo & ~LM);
+                        } else if (sizeof(Real) == 8) {
+                            const double en = phi64_in<KIND>(q, n, in), eo = phi64_in<KIND>(q, o, io);
+                            term[u] = en - eo;
+                        } else {
+                            term[u] = (double)(phi32<KIND>(q, (float)n, in) - phi32<KIND>(q, (float)o, io));
+                        }
+                    }
+                    if (!WELL) {
+                        if (H == 1) {
+#pragma unroll
+                            for (uint32_t u = 0; u < KP; ++u) side += term[u];
+                        } else {
+                            // lanes whose h is at least 1, 2, 4
+                            constexpr uint64_t F1 = G == 16 ? 0xfefefefefefefefeull : 0xaaaaaaaaaaaaaaaaull;
+                            constexpr uint64_t F2 = 0xfcfcfcfcfcfcfcfcull, F4 = 0xf0f0f0f0f0f0f0f0ull;
+                            const bool far1 = (any & F1) != 0, far2 = (any & F2) != 0, far4 = (any & F4) != 0;
+                            dEL = add_side<G, 0, KP>(dEL, term, far1, far2, far4);
+                            dER = add_side<G, H, KP>(dER, term, far1, far2, far4);
+                        }
+                    }
+                    if (H * KP >= COOP_W) break;
+                    k0 += H * KP;
+                    // the last partner of a side inside somewhere: the next ones
+                    constexpr uint64_t LAST = G == 16 ? 0x8080808080808080ull : G == 4 ? 0xaaaaaaaaaaaaaaaaull : ~0ull;
+                    if (k0 >= c.w || (last_in & LAST) == 0) break;
+#pragma unroll
+                    for (uint32_t u = 0; u < KP; ++u) xj[u] = partner(k0 + h * KP + u + 1);
+                }
+                if (H == 1 && !WELL) {
+                    dEL = from_lane<G, 0>(side);
+                    dER = from_lane<G, H>(side);
+                }
+                const double dE = WELL ? -q.p1 * (double)wL + -q.p1 * (double)wR : dEL + dER;
+                bool accd;
+                if (sizeof(Real) == 8) {
+                    const double e = -dE * beta;
+                    accd = go & ((dE <= 0.0) | (e > rn.y + 1e-4));
+                    const bool unsure = go & !accd & !(e < rn.y - 1e-4);
+                    if (__any(unsure)) accd = accd || (unsure && exp_apart(e) > u32o(rndw[ri]));
+                } else {
+                    accd = go & ((dE <= 0.0) | ((double)fexp(-betaf * (float)dE) > rn.y));
+                }
+                // the position and its periodic images: one lane each
+                const double xs = accd ? xn : xi;
+                if (t - put0 < putn) c.R[putb + t] = xs + putL;
+                if (a.acclog && g == 0) a.acclog[log_off + (uint64_t)(soff + sw) * c.N + i] = accd ? 1 : 0;
+                dUs += accd ? dE : 0.0;
+                acc += accd ? 1u : 0u;
+            }
+            __syncthreads();
+        }
+
+        // box-length trial (fav, src/jmmMCState.cpp:2161-2293)
+        VolProp vp{};
+        bool bad = false;
+        double vpart = 0.0, upart = 0.0;
+        if (npt) {
+            vp = sc.vp;
+            const bool last = c.per && b + 1 == c.B, von = vp.valid && act;
+            uint32_t t0 = 0, t1 = von ? half_of(size) : 0u;
+            const uint32_t tend = von ? size : 0u;
+            const int parts = smax >= HALF_MIN ? 2 : 1;
+#pragma unroll 1
+            for (int part = 0; part < parts; ++part) {
+                constexpr int NF = sizeof(Real) == 4 && !WELL ? 2 : 1;
+                double s[NF] = {};
+                block_sum<G, NF>(c, start, size, t0, t1, a0, gapR, g, work, s,
+                                 [&](uint32_t k, uint32_t t, double xi, double xj, bool run, double (&v)[NF]) {
+                                     const double xis = xi * vp.sc;
+                                     double xjs = xj * vp.sc;
+                                     if (run && last && t + k >= size) xjs = c.R[c.wg + t + k - size] * vp.sc + vp.Lp;
+                                     const double d0 = xj - xi, d1 = xjs - xis;
+                                     const bool hit = (k == 1) & run & (d1 < gmin);
+                                     bad = bad | hit;
+                                     const bool in0 = inside64<KIND>(q, d0), in1 = inside64<KIND>(q, d1);
+                                     if constexpr (sizeof(Real) == 8) {
+                                         v[0] = phi64_in<KIND>(q, d1, in1) - phi64_in<KIND>(q, d0, in0);
+                                         return !(hit | ((d0 > q.rc) & (d1 > q.rc)));
+                                     } else if constexpr (WELL) {
+                                         v[0] = in1 ? 1.0 : 0.0;
+                                         return in1 & !hit;
+                                     } else {
+                                         float e0;
+                                         v[0] = (double)box_term32<KIND>(q, vp.bk, (float)d0, (float)d1, in0, in1, e0);
+                                         v[1] = (double)e0;
+                                         return (in0 | in1) & !hit;
+                                     }
+                                 });
+                vpart += WELL ? -q.p1 * s[0] : s[0];
+                if constexpr (NF == 2) upart += s[1];
+                t0 = t1;
+                t1 = tend;
+            }
+        }
+        {
+            if (act && g == 0) {
+                blk[b] = dUs;
+                if (npt) {
+                    blk[c.B + b] = vpart;
+                    blk[2 * c.B + b] = upart;
+                }
+            }
+            const uint32_t par = (uint32_t)sweep & 1u;
+            // the wave's accepted trials, a bit of the blocks' counts at a time
+            uint32_t wacc = 0;
+            for (uint32_t m = 0; m < 32; ++m) {
+                const uint32_t rest = act && g == 0 ? acc >> m : 0u;
+                if (!__any(rest != 0)) break;
+                wacc += (uint32_t)__popcll(__ballot(rest & 1u)) << m;
+            }
+            if (lane == 0 && wacc) atomicAdd(&sc.acc[par], wacc);
+            if (__any(bad) && lane == 0) sc.bad[par] = 1u;
+            __syncthreads();
+            double v[3] = {0.0, 0.0, 0.0};
+            if (npt) {
+                chain_sum<3>(blk, c.B, sc, v);
+            } else {
+                double v1[1];
+                chain_sum<1>(blk, c.B, sc, v1);
+                v[0] = v1[0];
+            }
+            acc = sc.acc[par];
+            bad = sc.bad[par] != 0;
+            if (tid == 0) sc.acc[par ^ 1u] = sc.bad[par ^ 1u] = 0;
+            U = U + v[0];
+            vpart = v[1];
+            if (WELL) vpart = vpart - U;
+            else if (sizeof(Real) == 4 && npt && vp.valid && !bad) U = v[2];
+        }
+        acc_total += acc;
+        uint32_t accv = 0;
+        if (npt) {
+            ++n_vt;
+            if (vp.valid && !bad && vol_accept(vpart, vp.dL, vp.lns, P, beta, vp.jac, vp.u)) {
+                for (uint32_t t = g; t < size; t += G) c.R[a0 + t] = c.R[a0 + t] * vp.sc;
+                L = vp.Lp;
+                U = U + vpart;
+                accv = 1;
+                ++n_av;
+                __syncthreads();
+                fill_ghosts(c, tid, T, L);
+            }
+        }
+        __syncthreads();
+
+        // drift guard (ECheck, src/jmmMCState.cpp:1965-2095), always FP64
+        if (eci && (sweep + 1) % eci == 0) {
+            double s[1] = {0.0};
+            block_sum<G, 1>(c, start, size, 0u, size, a0, gapR, g, work, s,
+                            [&](uint32_t, uint32_t, double xi, double xj, bool, double (&v)[1]) {
+                                const double d = xj - xi;
+                                v[0] = phi64<KIND>(q, d);
+                                return !(d > q.rc);
+                            });
+            if (act && g == 0) blk[b] = s[0];
+            __syncthreads();
+            double v[1];
+            chain_sum<1>(blk, c.B, sc, v);
+            const double dr = fabs(v[0] - U);
+            if (dr > mdrift) mdrift = dr;
+            U = v[0];
+            ++n_rc;
+            __syncthreads();
+        }
+
+        double Ws = 0.0, Hs = 0.0;
+        if (a.sW) {
+            double s[2] = {0.0, 0.0};
+            block_sum<G, 2>(c, start, size, 0u, size, a0, gapR, g, work, s,
+                            [&](uint32_t, uint32_t, double xi, double xj, bool, double (&v)[2]) {
+                                const double d = xj - xi;
+                                virial64<KIND>(q, d, v[0], v[1]);
+                                // inside nothing adds nothing (strict cutoffs)
+                                const bool in = inside64<KIND>(q, d);
+                                v[0] = in ? v[0] : 0.0;
+                                v[1] = in ? v[1] : 0.0;
+                                return !(d > q.rc);
+                            });
+            if (act && g == 0) {
+                blk[b] = s[0];
+                blk[c.B + b] = s[1];
+            }
+            __syncthreads();
+            double v[2];
+            chain_sum<2>(blk, c.B, sc, v);
+            Ws = v[0];
+            Hs = v[1];
+            __syncthreads();
+        }
+        if (tid == 0) {
+            const uint64_t row = (uint64_t)(soff + sw) * a.n_chains + ic;
+            a.sU[row] = U;
+            a.sL[row] = L;
+            a.sA[row] = make_uint2(acc, accv);
+            if (a.sW) {
+                a.sW[row] = Ws;
+                a.sH[row] = Hs;
+            }
+        }
+    }
+
+    if (act && g == 0) {
+        atomicAdd(&sc.wall, n_wall);
+        atomicAdd(&sc.core, n_core);
+    }
+    atomicAdd(&sc.terms, n_terms);
+    __syncthreads();
+    if (tid == 0) {
+        DevState &o = a.states[ic];
+        o.L = L;
+        o.U = U;
+        o.sweep = sweep;
+        o.cnt[0] += (uint64_t)a.n_sweeps * c.N;
+        o.cnt[1] += acc_total;
+        o.cnt[2] += sc.wall;
+        o.cnt[3] += sc.core;
+        o.cnt[4] += sc.terms;
+        o.cnt[5] += n_vt;
+        o.cnt[6] += n_av;
+        o.cnt[7] += n_rc;
+        o.max_drift = mdrift;
+    }
+    double *xw = a.x + ch.x_off;
+    for (uint32_t t = g; t < size; t += G) xw[start + t] = c.R[a0 + t];
+}
+
+// The layout of a chain: lanes per block by the block count (coop_lanes), and
+// with few of them two partners per lane at once, so that one pass over the
+// partners is the usual case.
+template <typename Real, int KIND>
+__device__ __forceinline__ void run_coop_kind(const SweepArgs &a, uint32_t ic, double *smem, CoopScratch &sc,
+                                              uint32_t soff, uint32_t lanes, uint32_t w)
+{
+    if (lanes == 16) run_coop<Real, KIND, 16, 1>(a, ic, smem, sc, soff);
+    else if (KIND != POT_HRSW && w > 2 && lanes == 4) run_coop<Real, KIND, 4, 2>(a, ic, smem, sc, soff);
+    else if (lanes == 4) run_coop<Real, KIND, 4, 1>(a, ic, smem, sc, soff);
+    else run_coop<Real, KIND, 2, 2>(a, ic, smem, sc, soff);
+}
+
+template <typename Real>
+__global__ void __launch_bounds__(COOP_T) k_sweep_coop(SweepArgs a)
+{
+    extern __shared__ __align__(16) double smem[];
+    __shared__ CoopScratch sc;
+    const uint32_t soff = a.ctrl->sample_off;
+    const uint32_t ic = a.plain_list[blockIdx.x];
+    const DevChain &ch = a.chains[ic];
+    const uint32_t lanes = coop_lanes(ch.B);
+    switch (ch.kind) {
+    case POT_LJ:
+        run_coop_kind<Real, POT_LJ>(a, ic, smem, sc, soff, lanes, ch.w);
+        break;
+    case POT_HARMONIC:
+        run_coop_kind<Real, POT_HARMONIC>(a, ic, smem, sc, soff, lanes, ch.w);
+        break;
+    case POT_HRSW:
+        run_coop_kind<Real, POT_HRSW>(a, ic, smem, sc, soff, lanes, ch.w);
+        break;
+    default:
+        run_coop_kind<Real, POT_YUKAWA>(a, ic, smem, sc, soff, lanes, ch.w);
+        break;
     }
 }
 
@@ -1650,7 +2303,7 @@ __device__ __forceinline__ void run_segment(const SegArgs &g, const DevSeg &sg, 
         uint32_t bad = 0;
         double vpart = 0.0, upart = 0.0;
         if (npt) {
-            vp = vol_propose(ch, L, sweep);
+            vp = vol_propose<Real>(ch, L, sweep);
             const bool last = per && r + 1 == Bs && s + 1 == S, von = vp.valid && act;
             auto wrap = [&](uint32_t m) { return seg_load(&g.pub_head[(uint64_t)sg.first * W + m]); };
             const uint32_t h = half_of(size);
@@ -1926,7 +2579,7 @@ __device__ void run_plain(const SweepArgs &a, uint32_t ic, double *smem, uint32_
         uint32_t accv = 0;
         if (npt) {
             ++n_vt;
-            const VolProp vp = vol_propose(ch, L, sweep);
+            const VolProp vp = vol_propose<double>(ch, L, sweep);
             if (vp.valid) {
                 uint32_t bad = 0;
                 double u0;
@@ -2335,6 +2988,31 @@ hipError_t launch_batched(const SweepArgs &a, int fp32, int T, int gx, uint32_t 
     const void *fn = batched_kernel(fp32, T, gx);
     void *args[] = {(void *)&a};
     return hipLaunchKernel(fn, dim3(grid), dim3(T), args, lds, s);
+}
+
+size_t coop_lds(const DevChain &c)
+{
+    const size_t G = coop_lanes(c.B), T = (c.B * G + 63) / 64 * 64;
+    // the image and the block sums, then the random numbers (20 bytes for each
+    // of two positions a lane) or the pair terms (two fields a lane and partner)
+    const size_t rnd = T * 2 * 20 + 8, terms = T * c.w * 2 * sizeof(double);
+    return sizeof(double) * ((size_t)c.lds_len + 3 * c.B) + std::max(rnd, terms);
+}
+
+uint32_t coop_threads(const DevChain &c)
+{
+    return (c.B * coop_lanes(c.B) + 63) / 64 * 64;
+}
+
+const void *coop_kernel(int fp32)
+{
+    return fp32 ? (const void *)k_sweep_coop<float> : (const void *)k_sweep_coop<double>;
+}
+
+hipError_t launch_coop(const SweepArgs &a, int fp32, uint32_t grid, uint32_t threads, size_t lds, hipStream_t s)
+{
+    void *args[] = {(void *)&a};
+    return hipLaunchKernel(coop_kernel(fp32), dim3(grid), dim3(threads), args, lds, s);
 }
 
 const void *plain_kernel(int gx)

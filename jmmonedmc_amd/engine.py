@@ -80,7 +80,7 @@ class Engine:
 
     def __init__(self, chains, form="batched_fp32", device=0, sample_capacity=1024,
                  block_sweeps=100, wg_threads=0, use_graph=False, log_accepts=False,
-                 lds_budget=0, seg_lds=0, seg_lanes=0, sample_virial=False):
+                 lds_budget=0, seg_lds=0, seg_lanes=0, sample_virial=False, block_lanes=0):
         self.chains = list(chains)
         self.n = len(self.chains)
         self.form = nat.FORMS[form] if isinstance(form, str) else int(form)
@@ -95,6 +95,7 @@ class Engine:
         o.seg_lds = seg_lds
         o.seg_lanes = seg_lanes
         o.sample_virial = int(sample_virial)
+        o.block_lanes = block_lanes
         h = C.c_void_p()
         check(lib().jmm_create(specs, self.n, C.byref(o), C.byref(h)), "jmm_create")
         self.h = h
