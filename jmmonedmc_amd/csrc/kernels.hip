@@ -245,8 +245,9 @@ struct VolProp {
 };
 
 // Out of line: its FP64 log/exp/division temporaries would otherwise raise
-// the register count of the whole sweep loop.
-template <typename Real>
+// the register count of the whole sweep loop.  BOXK: with the scaling constants
+// of the LJ pair differences (two expm1), which only the FP32 LJ form reads.
+template <bool BOXK>
 __device__ __noinline__ VolProp vol_propose(const DevChain &ch, double L, uint64_t sweep)
 {
     uint32_t r[4];
@@ -271,7 +272,7 @@ __device__ __noinline__ VolProp vol_propose(const DevChain &ch, double L, uint64
     }
     v.valid = v.Lp > 0.0 && (!(ch.flags & F_PERIODIC) || v.Lp > ch.Lmin);
     v.bk.c12 = v.bk.c6 = 0.0f;
-    if (sizeof(Real) == 4) {
+    if (BOXK) {
         // s^-12 - 1 and s^-6 - 1 from expm1 of ln s: no cancellation
         const double a6 = ch.pot.e4 * ch.pot.sig6;
         v.bk.c12 = (float)(a6 * ch.pot.sig6 * expm1(-12.0 * v.lns));
@@ -281,29 +282,81 @@ __device__ __noinline__ VolProp vol_propose(const DevChain &ch, double L, uint64
 }
 
 
+// v + the value of the lane whose index differs in bit OFF, for values that
+// are equal within aligned groups of OFF lanes (the levels of a butterfly sum):
+// there a mirrored lane of the other half holds the partner's value, so the
+// levels inside a row are one data-parallel move and the two across rows a
+// swap, without the LDS round trip of a general shuffle.
+template <int OFF>
+__device__ __forceinline__ uint32_t xor_add(uint32_t v)
+{
+    if constexpr (OFF == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return r[0] + r[1];
+    } else if constexpr (OFF == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return r[0] + r[1];
+    } else {
+        // quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror, row_mirror
+        constexpr int ctrl = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x140;
+        return v + (uint32_t)__builtin_amdgcn_mov_dpp((int)v, ctrl, 0xf, 0xf, true);
+    }
+}
+
+template <int OFF>
+__device__ __forceinline__ double xor_add(double v)
+{
+    const uint32_t lo = (uint32_t)__double2loint(v), hi = (uint32_t)__double2hiint(v);
+    if constexpr (OFF == 16) {
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    } else if constexpr (OFF == 32) {
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    } else {
+        constexpr int ctrl = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x140;
+        return v + __hiloint2double(__builtin_amdgcn_mov_dpp((int)hi, ctrl, 0xf, 0xf, true),
+                                    __builtin_amdgcn_mov_dpp((int)lo, ctrl, 0xf, 0xf, true));
+    }
+}
+
+// One level of the sums below: lanes whose segment is longer than OFF add.
+template <int OFF, int ND, int NI>
+__device__ __forceinline__ void seg_level(double (&v)[ND], uint32_t (&k)[NI], uint32_t seg)
+{
+    const bool on = seg > (uint32_t)OFF;
+#pragma unroll
+    for (int m = 0; m < ND; ++m) {
+        const double s = xor_add<OFF>(v[m]);
+        v[m] = on ? s : v[m];
+    }
+#pragma unroll
+    for (int m = 0; m < NI; ++m) {
+        const uint32_t s = xor_add<OFF>(k[m]);
+        k[m] = on ? s : k[m];
+    }
+}
+
 // Sum over lane segments of size seg (seg <= T) whose first lane is base:
 // a power of two up to 64 with base a multiple of seg, or a multiple of 64
 // with base a multiple of 64 (whole waves).  Every lane of a segment
 // receives the same bits: the butterfly is symmetric in its operands, and
 // the cross-wave stage reads the segment's wave totals in a fixed order.
-// rd/ri: flat LDS scratch of (T/64)*ND doubles and (T/64)*NI words.
-template <int T, int ND, int NI>
+// rd/ri: flat LDS scratch of (T/64)*ND doubles and (T/64)*NI words.  TRAIL:
+// a barrier at the end, after which the scratch may be used again; without it
+// the caller has a barrier before the scratch's next use.
+template <int T, int ND, int NI, bool TRAIL = true>
 __device__ __forceinline__ void seg_allreduce(double (&v)[ND], uint32_t (&k)[NI], uint32_t seg,
                                               uint32_t base, double *rd, uint32_t *ri)
 {
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-#pragma unroll
-        for (int m = 0; m < ND; ++m) {
-            const double p = __shfl_xor(v[m], off);
-            if ((uint32_t)off < seg) v[m] += p;
-        }
-#pragma unroll
-        for (int m = 0; m < NI; ++m) {
-            const uint32_t p = __shfl_xor(k[m], off);
-            if ((uint32_t)off < seg) k[m] += p;
-        }
-    }
+    seg_level<1>(v, k, seg);
+    seg_level<2>(v, k, seg);
+    seg_level<4>(v, k, seg);
+    seg_level<8>(v, k, seg);
+    seg_level<16>(v, k, seg);
+    seg_level<32>(v, k, seg);
     if (T > 64) {
         const uint32_t tid = threadIdx.x, wv = tid >> 6;
         if ((tid & 63) == 0) {
@@ -328,7 +381,7 @@ __device__ __forceinline__ void seg_allreduce(double (&v)[ND], uint32_t (&k)[NI]
                 k[m] = acc;
             }
         }
-        __syncthreads();
+        if (TRAIL) __syncthreads();
     }
 }
 
@@ -336,19 +389,28 @@ __device__ __forceinline__ void seg_allreduce(double (&v)[ND], uint32_t (&k)[NI]
 template <typename V>
 __device__ __forceinline__ V wave_sum(V v)
 {
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off);
-    return v;
+    v = xor_add<1>(v);
+    v = xor_add<2>(v);
+    v = xor_add<4>(v);
+    v = xor_add<8>(v);
+    v = xor_add<16>(v);
+    return xor_add<32>(v);
 }
 
 // ------------------------------------------------------------ batched form
 
 template <int T>
 struct BatchedScratch {
-    double rd[(T / 64) * 4];
+    // no larger than before the proposals were shared: the image of a chain
+    // may leave 512 bytes of the LDS
+    static constexpr int NVP = T >= 1024 ? 1 : 2;
+    double rd[(T / 64) * 3];
+    VolProp vp[NVP];  // box-length proposals of chains of at least T / NVP blocks
     uint32_t ri[(T / 64) * 4];
     uint32_t item;
+    uint8_t need[T / 64];
 };
+static_assert(sizeof(BatchedScratch<256>) <= 512 && sizeof(BatchedScratch<512>) <= 512, "LDS left to a chain's image");
 
 template <typename Real, int KIND, int T>
 __device__ __forceinline__ void run_bundle_gx(const SweepArgs &a, const DevBundle &bd, BatchedScratch<T> &sc,
@@ -463,7 +525,7 @@ __device__ __forceinline__ void run_bundle_gx(const SweepArgs &a, const DevBundl
         uint32_t bad = 0;
         double vpart = 0.0, upart = 0.0;
         if (npt) {
-            vp = vol_propose<Real>(ch, L, sweep);
+            vp = vol_propose<sizeof(Real) == 4 && KIND == POT_LJ>(ch, L, sweep);
             if (vp.valid && act)
                 vpart = scaled_delta<Real, KIND>(q, vp.bk, gmin, X, N, per, L, vp.Lp, vp.sc, w, start,
                                                  start + size, 1, bad, upart);
@@ -582,6 +644,13 @@ __device__ __forceinline__ void fill_ghosts(const LdsChain &c, uint32_t r, uint3
         c.R[c.wg + c.B * c.Sp + m] = c.R[c.wg + m] + L;
         c.R[m] = c.R[tail + m] - L;
     }
+}
+
+// The periodic images of particle i at its new position x.
+__device__ __forceinline__ void put_images(const LdsChain &c, uint32_t i, double x, double L)
+{
+    if (i < c.wg) c.R[c.wg + c.B * c.Sp + i] = x + L;
+    if (i + c.wg >= c.N) c.R[i + c.wg - c.N] = x - L;
 }
 
 // The FP32 walks' keep-going test for one partner: inside the cutoff at the
@@ -1083,7 +1152,8 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
     const DevChain &sh = a.chains[__builtin_amdgcn_readfirstlane(a.slots[bd.slot0].chain)];
     const Pot q = sh.pot;
     const double gmin = sh.gmin;
-    const double max_step = ch.max_step;  // per chain: step adaptation may change it
+    // per chain: step adaptation may change it (2^-32: see the displacement)
+    const double step32 = ch.max_step * (1.0 / 4294967296.0);
     // per-chain fields as values: read once, not reloaded after every store
     // of the loops below (the compiler cannot rule out aliasing)
     const double beta = ch.beta;
@@ -1092,7 +1162,7 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
     const uint32_t chain_id = ch.chain_id;
     const uint64_t log_off = ch.log_off;
     const double P = ch.P;
-    const uint32_t eci = ch.eci;
+    const uint32_t eci = sh.eci;
 
     LdsChain c;
     c.R = smem + me.lds_off;
@@ -1116,6 +1186,12 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
     const uint32_t gapL = r == 0 ? 0u : c.Sp - (c.qb + (r - 1 < c.rem ? 1u : 0u));
     const uint32_t seg = act ? c.B : 1u;
     const bool leader = act && r == 0;
+    // waves none of whose particles has an image skip the image stores
+    const bool edges = c.per && __any(act && (start < c.wg || start + size + c.wg > c.N));
+    // a chain of several waves has its box-length proposal made by the first
+    // (some 200 to 400 instructions the others need not issue)
+    constexpr uint32_t WV = T / BatchedScratch<T>::NVP;
+    const bool waves = me.B >= WV;
 
     const double *xg = a.x + ch.x_off;
     for (uint32_t t = 0; t < size; ++t) c.R[a0 + t] = xg[start + t];
@@ -1126,14 +1202,21 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
     if (act) fill_ghosts(c, r, c.B, L);
     __syncthreads();
 
-    uint32_t n_tr = 0, n_wall = 0, n_core = 0, n_terms = 0;
+    uint32_t n_wall = 0, n_core = 0, n_terms = 0;
     uint32_t acc_total = 0, n_vt = 0, n_av = 0, n_rc = 0;
+    // sweeps to the next recompute
+    uint32_t to_eci = eci ? eci - (uint32_t)(sweep % eci) : 0u;
 
 #pragma unroll 1
     for (uint32_t sw = 0; sw < a.n_sweeps; ++sw, ++sweep) {
         double dUs = 0.0;
         uint32_t acc = 0;
         uint32_t w_md = 0, w_u = 0, w_next_md = 0, w_next_u = 0;
+        constexpr bool BOXK = sizeof(Real) == 4 && KIND == POT_LJ;
+        if (npt && waves && r < 64) {
+            const VolProp v = vol_propose<BOXK>(ch, L, sweep);
+            if (r == 0) sc.vp[me.lane_off / WV] = v;
+        }
 #pragma unroll 1
         for (uint32_t t = 0; t < bd.smax; ++t) {
             if (t < size) {
@@ -1153,12 +1236,13 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
                     w_md = w_next_md;
                     w_u = w_next_u;
                 }
-                const double a1 = u32o(w_md);
+                // ((u1 - 1/2) 2) max_step with u1 = (w + 1/2) 2^-32: the odd
+                // integer 2 (w - 2^31) + 1 times max_step 2^-32, the same
+                // product rounded once
                 const double u = u32o(w_u);
-                const double md = ((a1 - 0.5) * 2.0) * max_step;
+                const double md = fma((double)(int32_t)(w_md ^ 0x80000000u), 2.0, 1.0) * step32;
                 const double xi = c.R[my];
                 const double xn = xi + md;
-                ++n_tr;
                 double dE = 0.0;
                 // a window of one partner per side (the hard core keeps the
                 // second beyond the cutoff): the one-partner walk, which
@@ -1171,10 +1255,7 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
                                                              L, xi, xn, md, u, dE, n_terms, n_wall, n_core);
                 const double xs = accd ? xn : xi;
                 c.R[my] = xs;
-                if (c.per) {
-                    if (i < c.wg) c.R[c.wg + c.B * c.Sp + i] = xs + L;
-                    if (i + c.wg >= c.N) c.R[i + c.wg - c.N] = xs - L;
-                }
+                if (edges) put_images(c, i, xs, L);
                 dUs += accd ? dE : 0.0;
                 acc += accd ? 1u : 0u;
                 if (a.acclog) a.acclog[log_off + (uint64_t)(soff + sw) * c.N + i] = accd ? 1 : 0;
@@ -1188,7 +1269,8 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
         uint32_t bad = 0;
         double vpart = 0.0, upart = 0.0;
         if (npt) {
-            vp = vol_propose<Real>(ch, L, sweep);
+            if (waves) vp = sc.vp[me.lane_off / WV];
+            else vp = vol_propose<BOXK>(ch, L, sweep);
             auto wrap = [&](uint32_t m) { return c.R[c.wg + m]; };
             const bool last = c.per && r + 1 == c.B, von = vp.valid && act;
             // long blocks in two halves (half_of; a bundle's longest decides)
@@ -1209,7 +1291,12 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
         {
             double v[3] = {dUs, vpart, upart};
             uint32_t k2[2] = {acc, bad};
-            seg_allreduce<T, 3, 2>(v, k2, seg, me.lane_off, sc.rd, sc.ri);
+            if (eci) {
+                --to_eci;
+                const bool any = __any(act && to_eci == 0);
+                if ((tid & 63) == 0) sc.need[tid >> 6] = any ? 1 : 0;
+            }
+            seg_allreduce<T, 3, 2, false>(v, k2, seg, me.lane_off, sc.rd, sc.ri);
             U = U + v[0];
             vpart = v[1];
             acc = k2[0];
@@ -1227,22 +1314,29 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
         if (npt) {
             ++n_vt;
             if (vp.valid && !bad && vol_accept(vpart, vp.dL, vp.lns, P, beta, vp.jac, vp.u)) {
-                for (uint32_t t = 0; t < size; ++t) c.R[a0 + t] = c.R[a0 + t] * vp.sc;
                 L = vp.Lp;
+                // (idle lanes of the workgroup have size 0)
+                for (uint32_t t = 0; t < size; ++t) {
+                    const double xs = c.R[a0 + t] * vp.sc;
+                    c.R[a0 + t] = xs;
+                    if (edges) put_images(c, start + t, xs, L);
+                }
                 U = U + vpart;
                 accv = 1;
                 ++n_av;
             }
             __syncthreads();
-            // only the chain's own lanes: idle lanes of the workgroup carry no
-            // energy partials and so no valid decision
-            if (accv && act) fill_ghosts(c, r, c.B, L);
-            __syncthreads();
         }
 
+        // (constant length: the sums' scratch is read until here)
+        if (!npt && (eci || a.sW)) __syncthreads();
+
         // drift guard (ECheck, src/jmmMCState.cpp:1965-2095), always FP64
-        const int need = act && eci && ((sweep + 1) % eci == 0);
-        if (__syncthreads_or(need)) {
+        const bool need = act && eci && to_eci == 0;
+        uint32_t some = 0;
+        if (eci)
+            for (uint32_t m = 0; m < T / 64; ++m) some |= sc.need[m];
+        if (__builtin_amdgcn_readfirstlane(some)) {
             double Up = 0.0;
             if (need) {
                 for (uint32_t t = 0; t < size; ++t) {
@@ -1260,6 +1354,7 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
             double v[1] = {Up};
             uint32_t k1[1] = {0};
             seg_allreduce<T, 1, 1>(v, k1, seg, me.lane_off, sc.rd, sc.ri);
+            if (eci && to_eci == 0) to_eci = eci;
             if (need) {
                 const double dr = fabs(v[0] - U);
                 if (dr > mdrift) mdrift = dr;
@@ -1289,9 +1384,10 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
         }
     }
 
+    __syncthreads();
     {
         double vz[1] = {0.0};
-        uint32_t k4[4] = {n_tr, n_wall, n_core, n_terms};
+        uint32_t k4[4] = {size * a.n_sweeps, n_wall, n_core, n_terms};
         seg_allreduce<T, 1, 4>(vz, k4, seg, me.lane_off, sc.rd, sc.ri);
         if (leader) {
             DevState &o = a.states[ic];
@@ -1522,26 +1618,6 @@ __device__ __forceinline__ void block_sum(const LdsChain &c, uint32_t start, uin
     }
 }
 
-// v plus the value of the lane with one bit of its index flipped, for values
-// that are already equal within the smaller halves (so a mirrored lane of the
-// other half does): inside a row without an LDS round trip.
-template <int OFF, int ND>
-__device__ __forceinline__ void add_xor(double (&v)[ND])
-{
-#pragma unroll
-    for (int m = 0; m < ND; ++m) {
-        if constexpr (OFF >= 16) {
-            v[m] += __shfl_xor(v[m], OFF);
-        } else {
-            // quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror, row_mirror
-            constexpr int ctrl = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x140;
-            const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v[m]), ctrl, 0xf, 0xf, true);
-            const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v[m]), ctrl, 0xf, 0xf, true);
-            v[m] += __hiloint2double(hi, lo);
-        }
-    }
-}
-
 // Sums over the chain's blocks in the order of seg_allreduce (pairwise trees
 // over 64 blocks, then the trees in sequence), from per-block values in LDS:
 // one wave per 64 blocks, a block per lane; every lane of the workgroup
@@ -1554,12 +1630,13 @@ __device__ __forceinline__ void chain_sum(const double *blk, uint32_t B, CoopScr
         double p[ND];
 #pragma unroll
         for (int m = 0; m < ND; ++m) p[m] = l < top ? blk[m * B + q * 64 + l] : 0.0;
-        if (top > 1) add_xor<1>(p);
-        if (top > 2) add_xor<2>(p);
-        if (top > 4) add_xor<4>(p);
-        if (top > 8) add_xor<8>(p);
-        if (top > 16) add_xor<16>(p);
-        if (top > 32) add_xor<32>(p);
+        uint32_t none[1] = {0};
+        if (top > 1) seg_level<1>(p, none, 64);
+        if (top > 2) seg_level<2>(p, none, 64);
+        if (top > 4) seg_level<4>(p, none, 64);
+        if (top > 8) seg_level<8>(p, none, 64);
+        if (top > 16) seg_level<16>(p, none, 64);
+        if (top > 32) seg_level<32>(p, none, 64);
         if (l == 0)
 #pragma unroll
             for (int m = 0; m < ND; ++m) sc.grp[q][m] = p[m];
@@ -1601,7 +1678,8 @@ __device__ __forceinline__ void run_coop(const SweepArgs &a, uint32_t ic, double
     const uint32_t tid = threadIdx.x, T = blockDim.x, lane = tid & 63u;
     const DevChain &ch = a.chains[ic];
     const Pot q = ch.pot;
-    const double gmin = ch.gmin, max_step = ch.max_step, beta = ch.beta, P = ch.P;
+    const double gmin = ch.gmin, beta = ch.beta, P = ch.P;
+    const double step32 = ch.max_step * (1.0 / 4294967296.0);
     const float betaf = ch.betaf;
     const uint32_t key0 = (uint32_t)ch.seed, key1 = (uint32_t)(ch.seed >> 32);
     const uint32_t chain_id = ch.chain_id, eci = ch.eci;
@@ -1666,6 +1744,7 @@ __device__ __forceinline__ void run_coop(const SweepArgs &a, uint32_t ic, double
     fill_ghosts(c, tid, T, L);
     __syncthreads();
 
+    uint32_t to_eci = eci ? eci - (uint32_t)(sweep % eci) : 0u;  // sweeps to the next recompute
     // rejections per block, pair terms per lane
     uint32_t n_wall = 0, n_core = 0, n_terms = 0;
     uint32_t acc_total = 0, n_vt = 0, n_av = 0, n_rc = 0;
@@ -1678,7 +1757,7 @@ __device__ __forceinline__ void run_coop(const SweepArgs &a, uint32_t ic, double
         // the sweep's box-length proposal depends on L alone: the last wave
         // (the shortest blocks) prepares it
         if (npt && tid >= T - 64) {
-            const VolProp v = vol_propose<Real>(ch, L, sweep);
+            const VolProp v = vol_propose<sizeof(Real) == 4 && KIND == POT_LJ>(ch, L, sweep);
             if (lane == 0) sc.vp = v;
         }
 #pragma unroll 1
@@ -1694,7 +1773,7 @@ __device__ __forceinline__ void run_coop(const SweepArgs &a, uint32_t ic, double
                     for (int m = 0; m < 2; ++m) {
                         const double u = u32o(rr[2 * m + 1]);
                         const uint32_t at = b * 2 * G + 2 * g + m;
-                        rnd[at] = make_double2(((u32o(rr[2 * m]) - 0.5) * 2.0) * max_step,
+                        rnd[at] = make_double2(fma((double)(int32_t)(rr[2 * m] ^ 0x80000000u), 2.0, 1.0) * step32,
                                                sizeof(Real) == 8 ? (double)__logf((float)u) : u);
                         if (sizeof(Real) == 8) rndw[at] = rr[2 * m + 1];
                     }
@@ -1894,7 +1973,8 @@ __device__ __forceinline__ void run_coop(const SweepArgs &a, uint32_t ic, double
         __syncthreads();
 
         // drift guard (ECheck, src/jmmMCState.cpp:1965-2095), always FP64
-        if (eci && (sweep + 1) % eci == 0) {
+        if (eci && --to_eci == 0) {
+            to_eci = eci;
             double s[1] = {0.0};
             block_sum<G, 1>(c, start, size, 0u, size, a0, gapR, g, work, s,
                             [&](uint32_t, uint32_t, double xi, double xj, bool, double (&v)[1]) {
@@ -2303,7 +2383,7 @@ __device__ __forceinline__ void run_segment(const SegArgs &g, const DevSeg &sg, 
         uint32_t bad = 0;
         double vpart = 0.0, upart = 0.0;
         if (npt) {
-            vp = vol_propose<Real>(ch, L, sweep);
+            vp = vol_propose<sizeof(Real) == 4 && KIND == POT_LJ>(ch, L, sweep);
             const bool last = per && r + 1 == Bs && s + 1 == S, von = vp.valid && act;
             auto wrap = [&](uint32_t m) { return seg_load(&g.pub_head[(uint64_t)sg.first * W + m]); };
             const uint32_t h = half_of(size);
@@ -2579,7 +2659,7 @@ __device__ void run_plain(const SweepArgs &a, uint32_t ic, double *smem, uint32_
         uint32_t accv = 0;
         if (npt) {
             ++n_vt;
-            const VolProp vp = vol_propose<double>(ch, L, sweep);
+            const VolProp vp = vol_propose<false>(ch, L, sweep);
             if (vp.valid) {
                 uint32_t bad = 0;
                 double u0;
