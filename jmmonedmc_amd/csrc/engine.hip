@@ -264,6 +264,8 @@ struct Group {
     int gx = 0;
     int coop = 0;             // cooperative form: n_items chains in d_list
     uint32_t threads = 0;     // lanes per workgroup (cooperative form)
+    int waves = 2;            // batched kernel: waves per SIMD
+    int aside = 0;            // launched beside the first group, on the second stream
     uint32_t n_items = 0;     // bundles (batched) or chains (plain)
     uint32_t grid = 0;
     size_t lds = 0;
@@ -277,6 +279,10 @@ struct Group {
 // FP32: 1024 chains of 64 (8 waves per CU) 17.9 -> 10.6, 2048 (16) 17.9 -> 26.9;
 // 256 of 250 (8) 17.5 -> 11.2, 512 (16) 17.7 -> 22.0.
 constexpr uint64_t COOP_WAVES = 8;
+
+// LDS that a batched workgroup takes beside its bundle's image: at most 512
+// bytes, and what the allocation is rounded up by.
+constexpr size_t BATCHED_STATIC = 2560;
 
 // Phases of a sweep times the partners of a trial, by which chains end.
 static uint64_t chain_cost(const DevChain &c) { return (uint64_t)c.smax * (c.w + 2); }
@@ -296,6 +302,9 @@ static bool coop_gains(const DevChain &c)
 struct jmm_engine {
     int n = 0, form = 0, device = 0, T = 256;
     hipStream_t stream = nullptr;
+    // a second queue for a group that runs beside the first (launch_block)
+    hipStream_t stream2 = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     std::vector<jmm_chain_spec> specs;
     std::vector<DevChain> hch;          // internal order
     std::vector<uint32_t> int_of_ext, ext_of_int;
@@ -383,10 +392,19 @@ int fold_events(jmm_engine *e, bool all)
 
 int launch_block(jmm_engine *e, uint32_t m)
 {
+    // a group on the second stream starts after what the first has queued
+    // (the block before, reads, uploads) and is joined after its launch
+    bool fork = false;
+    for (const Group &G : e->grp) fork = fork || (G.aside && G.n_items);
+    if (fork) {
+        HIPCHK(hipEventRecord(e->ev_fork, e->stream));
+        HIPCHK(hipStreamWaitEvent(e->stream2, e->ev_fork, 0));
+    }
     for (size_t g = 0; g < e->grp.size(); ++g) {
         Group &G = e->grp[g];
         if (!G.n_items) continue;
-        HIPCHK(launch_begin(&e->d_ctrl[g], m, e->stream));
+        hipStream_t s = G.aside ? e->stream2 : e->stream;
+        HIPCHK(launch_begin(&e->d_ctrl[g], m, s));
         SweepArgs a{};
         a.chains = e->d_chains;
         a.states = e->d_states;
@@ -410,8 +428,11 @@ int launch_block(jmm_engine *e, uint32_t m)
         } else if (G.coop) {
             HIPCHK(launch_coop(a, e->form == JMM_FORM_BATCHED_FP32, G.grid, G.threads, G.lds, e->stream));
         } else {
-            HIPCHK(launch_batched(a, e->form == JMM_FORM_BATCHED_FP32, e->T, G.gx, G.grid, G.lds,
-                                  e->stream));
+            HIPCHK(launch_batched(a, e->form == JMM_FORM_BATCHED_FP32, e->T, G.gx, G.waves, G.grid, G.lds, s));
+        }
+        if (G.aside) {
+            HIPCHK(hipEventRecord(e->ev_join, s));
+            HIPCHK(hipStreamWaitEvent(e->stream, e->ev_join, 0));
         }
     }
     if (e->n_segs) {
@@ -567,6 +588,7 @@ int jmm_destroy(jmm_engine *e)
     if (!e) return 0;
     (void)hipSetDevice(e->device);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
+    if (e->stream2) (void)hipStreamSynchronize(e->stream2);
     if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
     if (e->graph) (void)hipGraphDestroy(e->graph);
     for (auto &p : e->ev) {
@@ -607,6 +629,9 @@ int jmm_destroy(jmm_engine *e)
         (void)hipFree(G.d_bundles);
         (void)hipFree(G.d_list);
     }
+    if (e->ev_fork) (void)hipEventDestroy(e->ev_fork);
+    if (e->ev_join) (void)hipEventDestroy(e->ev_join);
+    if (e->stream2) (void)hipStreamDestroy(e->stream2);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
     return 0;
@@ -661,6 +686,9 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
     }
     int lds_max = 0;
     CREATE_CHK(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, o.device));
+    int lds_cu = 0;
+    CREATE_CHK(hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, o.device));
+    lds_cu = std::max(lds_cu, lds_max);
     int n_cu = 0;
     CREATE_CHK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, o.device));
 
@@ -862,22 +890,62 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
             std::stable_sort(bv.begin(), bv.end(), [&](const DevBundle &a, const DevBundle &b) {
                 return bundle_cost(a, e->hch, slots) > bundle_cost(b, e->hch, slots);
             });
-            Group G;
-            G.gx = g;
-            G.n_items = (uint32_t)bv.size();
-            size_t maxd = 0;
-            for (auto &b : bv) maxd = std::max<size_t>(maxd, b.lds_doubles);
-            G.lds = g ? 0 : maxd * sizeof(double);
-            const void *fn = batched_kernel(e->form == JMM_FORM_BATCHED_FP32, e->T, g);
-            if (int rc = set_lds_attr(fn, G.lds)) return bail(rc);
-            int occ = 0;
-            CREATE_CHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, e->T, G.lds));
-            if (occ < 1) occ = 1;
-            G.grid = std::min<uint32_t>(G.n_items, (uint32_t)(occ * n_cu));
-            e->grp.push_back(G);  // owned by the engine from here: destroy releases it
-            Group &Gb = e->grp.back();
-            if (int rc = dalloc(&Gb.d_bundles, Gb.n_items)) return bail(rc);
-            CREATE_CHK(hipMemcpy(Gb.d_bundles, bv.data(), sizeof(DevBundle) * Gb.n_items, hipMemcpyHostToDevice));
+            // Three waves per SIMD need workgroups of at most a third of the
+            // CU's LDS. A launch allocates its largest bundle's image for
+            // every workgroup, so where some bundles are larger they get a
+            // launch of their own, beside the others' on a second stream, and
+            // the others are held to half of what one of them leaves of a CU:
+            // 100 sweeps of 4096 mixed chains of 32 to 8192 8.45 -> 7.19 ms
+            // (the larger ones with two waves' registers: 8.6, a CU then
+            // holds only one of the others beside them; a smaller share for
+            // the others, 40 or 36 KB of 45: 7.37, 7.59).
+            const int fp32 = e->form == JMM_FORM_BATCHED_FP32;
+            const bool may3 = !g && e->T == 256 && bv.size() > 2 * (size_t)n_cu;
+            const size_t share = (size_t)lds_cu / 3 - BATCHED_STATIC;
+            size_t limit = 0, largest = 0;
+            for (auto &b : bv) largest = std::max<size_t>(largest, b.lds_doubles * sizeof(double));
+            if (may3) {
+                const size_t with = largest + 3 * BATCHED_STATIC;
+                const size_t half = (size_t)lds_cu > with ? ((size_t)lds_cu - with) / 2 : 0;
+                limit = largest > share && half >= share / 2 ? half : share;
+            }
+            std::vector<DevBundle> part[2];
+            for (auto &b : bv) part[b.lds_doubles * sizeof(double) > limit ? 0 : 1].push_back(b);
+            // two launches only where the smaller bundles are the most of the work
+            double cost[2] = {0.0, 0.0};
+            for (int p = 0; p < 2; ++p)
+                for (auto &b : part[p]) cost[p] += bundle_cost(b, e->hch, slots);
+            if (!part[0].empty() && (part[1].size() <= 2 * (size_t)n_cu || cost[1] < cost[0])) {
+                part[0] = bv;
+                part[1].clear();
+            }
+            const bool both = !part[0].empty() && !part[1].empty();
+            for (int p = 0; p < 2; ++p) {
+                if (part[p].empty()) continue;
+                Group G;
+                G.gx = g;
+                G.waves = p == 1 || both ? 3 : 2;
+                G.aside = both && p == 1;
+                G.n_items = (uint32_t)part[p].size();
+                size_t maxd = 0;
+                for (auto &b : part[p]) maxd = std::max<size_t>(maxd, b.lds_doubles);
+                G.lds = g ? 0 : maxd * sizeof(double);
+                const void *fn = batched_kernel(fp32, e->T, g, G.waves);
+                if (int rc = set_lds_attr(fn, G.lds)) return bail(rc);
+                int occ = 0;
+                CREATE_CHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, e->T, G.lds));
+                if (occ < 1) occ = 1;
+                G.grid = std::min<uint32_t>(G.n_items, (uint32_t)(occ * n_cu));
+                e->grp.push_back(G);  // owned by the engine from here: destroy releases it
+                Group &Gb = e->grp.back();
+                if (int rc = dalloc(&Gb.d_bundles, Gb.n_items)) return bail(rc);
+                CREATE_CHK(hipMemcpy(Gb.d_bundles, part[p].data(), sizeof(DevBundle) * Gb.n_items, hipMemcpyHostToDevice));
+            }
+            if (both) {
+                CREATE_CHK(hipStreamCreateWithFlags(&e->stream2, hipStreamNonBlocking));
+                CREATE_CHK(hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming));
+                CREATE_CHK(hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming));
+            }
         }
     }
     // segmented chains: one launch, one workgroup per segment, all resident

@@ -153,8 +153,9 @@ struct HistArgs {
 
 namespace jmm {
 hipError_t launch_begin(Ctrl *c, uint32_t n, hipStream_t s);
-const void *batched_kernel(int fp32, int T, int gx);
-hipError_t launch_batched(const SweepArgs &a, int fp32, int T, int gx, uint32_t grid, size_t lds,
+// waves: per SIMD, 2 or (T = 256 in LDS) 3
+const void *batched_kernel(int fp32, int T, int gx, int waves);
+hipError_t launch_batched(const SweepArgs &a, int fp32, int T, int gx, int waves, uint32_t grid, size_t lds,
                           hipStream_t s);
 // Cooperative form: one chain per workgroup of at most COOP_T lanes (512: two
 // waves per SIMD, so 256 registers; 1024 lanes with 128 spilled), 16, 4 or 2

@@ -17,11 +17,6 @@
 //   k_begin          resets a work queue and advances the sample row.
 #include "kernels.h"
 
-// Occupancy target of the batched kernels (waves per SIMD); bounds VGPRs.
-#ifndef JMM_WAVES_PER_EU
-#define JMM_WAVES_PER_EU 2
-#endif
-
 namespace jmm {
 
 __device__ __forceinline__ bool nbpos(const double *X, int64_t j, int64_t N, bool per, double L,
@@ -1411,11 +1406,16 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
 }
 
 // Persistent kernel, one instantiation per (precision, workgroup size,
-// memory mode): every workgroup pulls bundles from one queue (all potentials
-// together, longest first) until it is empty; all waves of a workgroup leave
-// together when the queue is drained.  The potential is uniform per bundle.
-template <typename Real, int T, bool GX>
-__global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(JMM_WAVES_PER_EU)))
+// memory mode, waves per SIMD): every workgroup pulls bundles from one queue
+// (all potentials together, longest first) until it is empty; all waves of a
+// workgroup leave together when the queue is drained.  The potential is
+// uniform per bundle.  W waves per SIMD bound the registers: 2 (256, 193 used),
+// or 3 for 256 lanes (168, 21 spilled outside the phases), which hides more of
+// the phases' latency where there are bundles for it: 4096 mixed chains of 32 to
+// 4000, FP32, 55.0 us a sweep with 2, 44.6 with 3 (4: 128 registers, 269
+// spilled, 59.5); bundles that fit at 2 lose 1 to 2 % to the spills.
+template <typename Real, int T, bool GX, int W>
+__global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(W)))
 k_sweep_batched(SweepArgs a)
 {
     extern __shared__ double smem[];
@@ -3047,25 +3047,26 @@ hipError_t launch_begin(Ctrl *c, uint32_t n, hipStream_t s)
 }
 
 template <typename Real>
-static const void *pick_shape(int T, int gx)
+static const void *pick_shape(int T, int gx, int waves)
 {
-    if (T == 1024) return gx ? (const void *)k_sweep_batched<Real, 1024, true>
-                             : (const void *)k_sweep_batched<Real, 1024, false>;
-    if (T == 512) return gx ? (const void *)k_sweep_batched<Real, 512, true>
-                            : (const void *)k_sweep_batched<Real, 512, false>;
-    return gx ? (const void *)k_sweep_batched<Real, 256, true>
-              : (const void *)k_sweep_batched<Real, 256, false>;
+    if (T == 1024) return gx ? (const void *)k_sweep_batched<Real, 1024, true, 2>
+                             : (const void *)k_sweep_batched<Real, 1024, false, 2>;
+    if (T == 512) return gx ? (const void *)k_sweep_batched<Real, 512, true, 2>
+                            : (const void *)k_sweep_batched<Real, 512, false, 2>;
+    if (gx) return (const void *)k_sweep_batched<Real, 256, true, 2>;
+    return waves == 3 ? (const void *)k_sweep_batched<Real, 256, false, 3>
+                      : (const void *)k_sweep_batched<Real, 256, false, 2>;
 }
 
-const void *batched_kernel(int fp32, int T, int gx)
+const void *batched_kernel(int fp32, int T, int gx, int waves)
 {
-    return fp32 ? pick_shape<float>(T, gx) : pick_shape<double>(T, gx);
+    return fp32 ? pick_shape<float>(T, gx, waves) : pick_shape<double>(T, gx, waves);
 }
 
-hipError_t launch_batched(const SweepArgs &a, int fp32, int T, int gx, uint32_t grid, size_t lds,
+hipError_t launch_batched(const SweepArgs &a, int fp32, int T, int gx, int waves, uint32_t grid, size_t lds,
                           hipStream_t s)
 {
-    const void *fn = batched_kernel(fp32, T, gx);
+    const void *fn = batched_kernel(fp32, T, gx, waves);
     void *args[] = {(void *)&a};
     return hipLaunchKernel(fn, dim3(grid), dim3(T), args, lds, s);
 }
