@@ -1043,7 +1043,9 @@ static int launch_hist_sample(jmm_engine *e)
     h.gnb = e->hs.gnb;
     uint64_t nmax = 1;
     for (const auto &c : e->hch) nmax = std::max<uint64_t>(nmax, c.N);
-    h.parts = (uint32_t)std::min<uint64_t>(64, (nmax + 255) / 256);
+    // a workgroup per tile; of engines with many chains as long as the parts of
+    // the longest (the others' return at once) stay within some ten rounds
+    h.parts = (uint32_t)std::min<uint64_t>((nmax + HIST_TILE - 1) / HIST_TILE, std::max<uint64_t>(64, 4096 / e->n));
     HIPCHK(launch_hist(h, e->stream));
     e->hist_samples++;
     return 0;
