@@ -2745,29 +2745,93 @@ __global__ void k_begin(Ctrl *c, uint32_t n)
 
 // ------------------------------------------------------- differentiation
 
+// pair_obs and the force over distance f = o[1] / d of one pair.  rsig = 1 / p1
+// (LJ's sigma, as the FP32 form rounds it).  The FP32 LJ and Yukawa pairs hold
+// four and two divisions, half of their instructions.  A quotient of two FP32
+// numbers lies at least 2^-49 of itself from the middle of two neighbours, so
+// a product in FP64 with a reciprocal good to a few 2^-53 rounds to the same
+// FP32 number as the division: FP32 estimates, each with two Newton steps in
+// FP64, give the same bits.  Two more steps from 1 / (float)d lead to 1 / d to
+// the last bits of FP64.  Outside (1e-4, 1e4), where d^6 or its reciprocal
+// could leave the estimate's range, for the other potentials and for FP64: the
+// divisions.
+template <int KIND, typename R>
+__device__ __forceinline__ void pair_obs_f(const Pot &q, double rsig, double d, const R sh[3], R o[6], double &f)
+{
+    if constexpr (sizeof(R) == 4 && (KIND == POT_LJ || KIND == POT_YUKAWA)) {
+        if (d > 1e-4 && d < 1e4) {
+            const float x = (float)d;
+            double r = (double)frcp(x);
+            if constexpr (KIND == POT_LJ) {
+                const float d3 = x * x * x, d6 = d3 * d3;
+                double r6 = (double)frcp(d6);
+                r6 = fma(fma(-(double)d6, r6, 1.0), r6, r6);
+                r6 = fma(fma(-(double)d6, r6, 1.0), r6, r6);
+                const float i6 = (float)r6 * q.sig6f, i12 = i6 * i6;
+                const float a12 = q.e4f * i12, a6 = q.e4f * i6;
+                o[0] = (a12 - a6) - sh[0];
+                o[1] = 12.0f * a12 - 6.0f * a6;
+                o[2] = (4.0f * i12 - 4.0f * i6) - sh[1];
+                o[3] = (float)((double)o[1] * rsig) - sh[2];
+                o[4] = 12.0f * (4.0f * i12) - 6.0f * (4.0f * i6);
+                o[5] = (float)((double)(144.0f * a12 - 36.0f * a6) * rsig);
+            } else {
+                r = fma(fma(-(double)x, r, 1.0), r, r);
+                r = fma(fma(-(double)x, r, 1.0), r, r);
+                const float e = expf(-q.p1f * x);
+                const float ed = (float)((double)e * r);
+                const float E = q.p0f * ed;
+                o[0] = E - sh[0];
+                o[1] = E * (q.p1f * x + 1.0f);
+                o[2] = ed - sh[1];
+                o[3] = -q.p0f * e - sh[2];
+                o[4] = ed * (q.p1f * x + 1.0f);
+                o[5] = -q.p1f * x * x * E;
+            }
+            r = fma(fma(-d, r, 1.0), r, r);
+            r = fma(fma(-d, r, 1.0), r, r);
+            f = (double)o[1] * r;
+            return;
+        }
+    }
+    pair_obs<KIND, R>(q, R(d), sh, o);
+    f = (double)o[1] / d;
+}
+
+// LDS of the observables kernel: the waves' sums, forces handed to the next
+// wave, and the edge's forces by wave.
+struct ObsScratch {
+    double red[16 * 6], next[16 * 64], edge[16 * 64];
+};
+
 // U, W and their parameter derivatives of one tile of a configuration
 // (particles [p0, p1): the pairs whose left member is in the tile) and dU/dx
 // of the tile's particles.  Pair arithmetic in Real, sums in FP64.
 // out = (U, W, dU/dtheta0, dU/dtheta1, dW/dtheta0, dW/dtheta1) of the tile.
 //
-// Bound by vector issue: about 16 pairs a side for the 20 sigma Yukawa
-// chains at density 0.8, each some 70 instructions (an FP32 exponential and
-// division or an FP64 division, and six FP64 sums) against 16 bytes of
-// memory per particle, so what matters is that every SIMD has waves to
-// issue from.  A particle per lane and tiles of OBS_TILE spread a long
-// configuration over the chip, where one workgroup each left 64
-// configurations of 65,536 on 64 of the 256 CUs with one wave per SIMD
-// (forward and backward of those through the autograd binding, FP32: 3.67 ms
-// with one workgroup each, 0.376 ms with tiles).
-// Neighbouring lanes read neighbouring positions (L1 hits); the left partners
-// are evaluated again for dU/dx (W only) rather than exchanged, which would
-// need a barrier per partner.
+// Bound by vector issue (every SIMD's issue slots are taken on the 20 sigma
+// Yukawa chains at density 0.8): about 16 pairs a side, each some 90
+// instructions, against 16 bytes of memory per particle.  Two things matter:
+// that every SIMD has waves to issue from (a particle per lane and tiles of
+// OBS_TILE over the chip: one workgroup each left 64 configurations of 65,536
+// on 64 of the 256 CUs with one wave per SIMD, 3.67 ms), and that each pair is
+// evaluated once.  A lane walks its right-hand partners; the partner at index
+// distance k gets the pair's force by a shift of the wave's lanes by k (in the
+// wave, or its next one by an LDS row at the end: no barrier in the walk).
+// Only pairs that cross the tile's left edge, or reach beyond 64 partners, are
+// evaluated again from the right; the edge's are spread over the waves by
+// index distance (left to the first wave they cost as much as both walks did:
+// it sits on the same SIMD in every workgroup).  The walk is uniform over the
+// wave with the next position loaded ahead.
+// The kernel, FP32: 64 Yukawa configurations of 65,536 314 us with both sides
+// walked, 244 with each pair once, 225 with the divisions of pair_obs_f and
+// tiles of 512; 1024 LJ chains of 1024 28 and 22 us.
 template <typename Real, int KIND>
 __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, double L, double sc, uint32_t p0,
-                                        uint32_t p1, double *out, double *grad)
+                                        uint32_t p1, double *out, double *grad, ObsScratch &sm)
 {
-    __shared__ double red[16 * 6];
-    const uint32_t tid = threadIdx.x;
+    double *red = sm.red, *next = sm.next, *edge = sm.edge;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, waves = blockDim.x >> 6;
     const Pot q = ch.pot;
     const uint32_t N = ch.N;
     // a compressed configuration (sc < 1) may hold gaps below the hard core:
@@ -2775,47 +2839,89 @@ __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, dou
     const uint32_t w = sc < 1.0 ? min(ch.nbn_lim, N > 0 ? N - 1 : 0u) : ch.w;
     const bool per = (ch.flags & F_PERIODIC) != 0;
     const Real sh[3] = {Real(ch.sh[0]), Real(ch.sh[1]), Real(ch.sh[2])};
+    const double rsig = 1.0 / (double)q.p1f;
     double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (uint32_t i = p0 + tid; i < p1; i += blockDim.x) {
+    for (uint32_t t0 = p0; t0 < p1; t0 += blockDim.x) {
+        const uint32_t i = t0 + tid;
         // positions of the configuration scaled by sc to length L: x_j sc,
-        // periodic images x_j sc -+ L
-        const double xi = X[i] * sc;
-        double g = 0.0;
-        for (uint32_t k = 1; k <= w; ++k) {
-            const uint32_t j = i + k;
-            double xj;
-            if (j < N) xj = X[j] * sc;
-            else if (per) xj = X[j - N] * sc + L;
-            else break;
-            const double d = xj - xi;
-            if (d > q.rc) break;
-            // a rescaled configuration can overlap hard cores: infinite energy
-            if ((KIND == POT_HRSW && d < q.p0) || (KIND == POT_YUKAWA && d < q.p2)) {
-                acc[0] += INFINITY;
-                continue;
-            }
-            if (!inside64<KIND>(q, d)) continue;
-            Real o[6];
-            pair_obs<KIND, Real>(q, Real(d), sh, o);
-#pragma unroll
-            for (int m = 0; m < 6; ++m) acc[m] += (double)o[m];
-            g += (double)o[1] / d;
+        // periodic images x_j sc -+ L.  Lanes past the end stay on the last
+        // particle (j < 2N) and are never active.
+        const uint32_t ic = min(i, p1 - 1);
+        const double xi = X[ic] * sc;
+        bool active = i < p1;
+        double g = 0.0, gl = 0.0, gn = 0.0;
+        uint32_t j = ic + 1;
+        double off = 0.0;
+        if (j == N) {
+            j = 0;
+            off = L;
+            active = active && per;
         }
-        if (grad) {
-            for (uint32_t k = 1; k <= w; ++k) {
+        double xn = X[j] * sc + off;
+        for (uint32_t k = 1; k <= w; ++k) {
+            const double d = xn - xi;
+            active = active && !(d > q.rc);
+            if (!__ballot(active)) break;
+            const bool in = active && inside64<KIND>(q, d);
+            if (++j == N) {
+                j = 0;
+                off = L;
+                active = active && per;
+            }
+            xn = X[j] * sc + off;
+            double f = 0.0;
+            if (in) {
+                Real o[6];
+                pair_obs_f<KIND, Real>(q, rsig, d, sh, o, f);
+                // a rescaled configuration can overlap hard cores: infinite energy
+                if ((KIND == POT_HRSW && d < q.p0) || (KIND == POT_YUKAWA && d < q.p2)) {
+                    acc[0] += INFINITY;
+                } else {
+#pragma unroll
+                    for (int m = 0; m < 6; ++m) acc[m] += (double)o[m];
+                    g += f;
+                }
+            }
+            if (grad && k <= 64) {
+                const int from = (int)((lane - k) & 63u) << 2;
+                const double fl = __hiloint2double(__builtin_amdgcn_ds_bpermute(from, __double2hiint(f)),
+                                                   __builtin_amdgcn_ds_bpermute(from, __double2loint(f)));
+                if (lane >= k) gl += fl;
+                else gn += fl;
+            }
+        }
+        if (!grad) continue;
+        // pairs evaluated again: the force of the left-hand partners of
+        // particle m at index distances k0, k0 + step, ...
+        const auto left = [&](uint32_t m, uint32_t k0, uint32_t step) {
+            const double xm = X[m] * sc;
+            double s = 0.0;
+            for (uint32_t k = k0; k <= w; k += step) {
                 double xj;
-                if (k <= i) xj = X[i - k] * sc;
-                else if (per) xj = X[i + N - k] * sc - L;
+                if (k <= m) xj = X[m - k] * sc;
+                else if (per) xj = X[m + N - k] * sc - L;
                 else break;
-                const double d = xi - xj;
+                const double d = xm - xj;
                 if (d > q.rc) break;
                 if (!inside64<KIND>(q, d)) continue;
                 Real o[6];
-                pair_obs<KIND, Real>(q, Real(d), sh, o);
-                g -= (double)o[1] / d;
+                double f;
+                pair_obs_f<KIND, Real>(q, rsig, d, sh, o, f);
+                s += f;
             }
-            grad[i] = g;
+            return s;
+        };
+        next[tid] = gn;
+        edge[tid] = t0 + lane < p1 ? left(t0 + lane, lane + 1 + wave, waves) : 0.0;
+        __syncthreads();
+        if (wave) {
+            gl += next[tid - 64];
+            if (i < p1) gl += left(i, 65, 1);
+        } else {
+            for (uint32_t v = 0; v < waves; ++v) gl += edge[v * 64 + lane];
         }
+        if (i < p1) grad[i] = g - gl;
+        __syncthreads();
     }
 #pragma unroll
     for (int m = 0; m < 6; ++m) acc[m] = wave_sum(acc[m]);
@@ -2832,9 +2938,13 @@ __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, dou
 // One workgroup per tile: a.tile particles of a configuration, or the whole
 // configuration (a.tiles = nullptr), whose observables then go straight to
 // the caller's row; with tiles they go to a.part, and k_obs_sum adds them.
+// FP32: 64 registers, so that two workgroups of 1024 share a CU (27 -> 22 us
+// for 1024 chains of 1024).
 template <typename Real>
-__global__ void __launch_bounds__(1024) k_observables(ObsArgs a)
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 8 : 4)))
+k_observables(ObsArgs a)
 {
+    __shared__ ObsScratch sm;  // one for the four potentials
     uint32_t c, p0 = 0, part = 0;
     if (a.standalone) {
         c = blockIdx.x / a.parts;
@@ -2868,10 +2978,10 @@ __global__ void __launch_bounds__(1024) k_observables(ObsArgs a)
     if (a.part) out = a.part + (uint64_t)blockIdx.x * 6;
     else out = a.obs + (uint64_t)(a.row ? a.row[c] : c) * 6;
     switch (ch.kind) {
-    case POT_LJ: run_obs<Real, POT_LJ>(ch, X, L, sc, p0, p1, out, grad); break;
-    case POT_HARMONIC: run_obs<Real, POT_HARMONIC>(ch, X, L, sc, p0, p1, out, grad); break;
-    case POT_HRSW: run_obs<Real, POT_HRSW>(ch, X, L, sc, p0, p1, out, grad); break;
-    default: run_obs<Real, POT_YUKAWA>(ch, X, L, sc, p0, p1, out, grad); break;
+    case POT_LJ: run_obs<Real, POT_LJ>(ch, X, L, sc, p0, p1, out, grad, sm); break;
+    case POT_HARMONIC: run_obs<Real, POT_HARMONIC>(ch, X, L, sc, p0, p1, out, grad, sm); break;
+    case POT_HRSW: run_obs<Real, POT_HRSW>(ch, X, L, sc, p0, p1, out, grad, sm); break;
+    default: run_obs<Real, POT_YUKAWA>(ch, X, L, sc, p0, p1, out, grad, sm); break;
     }
 }
 
