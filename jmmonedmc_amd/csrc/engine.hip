@@ -1759,7 +1759,7 @@ int jmm_pair_observables_ws(const jmm_chain_spec *spec, int n_configs, const dou
     // holds their partial sums, else one workgroup each
     const uint64_t parts = obs_parts(s.N);
     if (parts > 1 && work_dev && work_doubles >= parts * 6 * (uint64_t)n_configs &&
-        parts * (uint64_t)n_configs <= 0x7fffffffull) {
+        parts * (uint64_t)n_configs <= 0xffffffffull / 64) {
         a.parts = (uint32_t)parts;
         a.tile = OBS_TILE;
         a.part = work_dev;

@@ -142,7 +142,8 @@ struct SegArgs {
 };
 
 // rho(x) and g(x) histograms of every chain's current configuration.
-// Histogram kernel: lanes of a workgroup, particles of a tile, 32-bit counters
+// Histogram kernel: lanes of a workgroup (HIST_TILE of them where a launch's
+// limit asks for it), particles of a tile, 32-bit counters
 // in LDS (64 KB: two workgroups per CU), and the longest chain whose tiles
 // cannot overflow them (HIST_TILE particles, N - 1 partners, both members).
 constexpr uint32_t HIST_T = 1024, HIST_TILE = 256, HIST_WORDS = 16384, HIST_N_LDS = 1u << 22;

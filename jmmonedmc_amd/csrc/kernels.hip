@@ -3119,7 +3119,7 @@ __global__ void __launch_bounds__(HIST_T) k_hist(HistArgs a)
     const DevChain &ch = a.chains[c];
     const uint32_t N = ch.N;
     // particles of a tile (short chains: more lanes per particle)
-    const uint32_t P = N <= 64 ? 64u : N <= 128 ? 128u : HIST_TILE, K = HIST_T / P;
+    const uint32_t P = N <= 64 ? 64u : N <= 128 ? 128u : HIST_TILE, K = blockDim.x / P;
     const uint32_t tiles = (N + P - 1) / P;
     if (part >= tiles) return;
     const bool per = (ch.flags & F_PERIODIC) != 0;
@@ -3143,7 +3143,7 @@ __global__ void __launch_bounds__(HIST_T) k_hist(HistArgs a)
             W = (uint32_t)min((int64_t)(HIST_WORDS / a.gnb), (f1 < f0 ? top : b1) - b0 + 1);
         }
         const uint32_t words = W * a.gnb;
-        for (uint32_t m = tid; m < words; m += HIST_T) hw[m] = 0;
+        for (uint32_t m = tid; m < words; m += blockDim.x) hw[m] = 0;
         __syncthreads();
         if (i < N) {
             const double xi = X[i];
@@ -3179,7 +3179,7 @@ __global__ void __launch_bounds__(HIST_T) k_hist(HistArgs a)
             }
         }
         __syncthreads();
-        for (uint32_t m = tid; m < words; m += HIST_T)
+        for (uint32_t m = tid; m < words; m += blockDim.x)
             if (const uint32_t v = hw[m]) atomicAdd(&g[(uint64_t)s0 * a.gnb + m], (unsigned long long)v);
         __syncthreads();
     }
@@ -3267,11 +3267,20 @@ hipError_t launch_plain(const SweepArgs &a, int gx, uint32_t grid, size_t lds, h
     return hipGetLastError();
 }
 
+// Lanes of a workgroup: as wanted, or fewer (whole waves, at least `least`)
+// where a launch of so many workgroups would pass its limit of 2^32 lanes.
+static uint32_t lanes_within(uint64_t groups, uint32_t want, uint32_t least)
+{
+    const uint64_t most = groups ? 0xffffffffull / groups / 64 * 64 : want;
+    return (uint32_t)std::max<uint64_t>(least, std::min<uint64_t>(want, most));
+}
+
 hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads,
                               hipStream_t s)
 {
-    if (fp32) hipLaunchKernelGGL(k_observables<float>, dim3(n_tiles), dim3(threads), 0, s, a);
-    else hipLaunchKernelGGL(k_observables<double>, dim3(n_tiles), dim3(threads), 0, s, a);
+    const uint32_t lanes = lanes_within(n_tiles, (uint32_t)threads, 64);
+    if (fp32) hipLaunchKernelGGL(k_observables<float>, dim3(n_tiles), dim3(lanes), 0, s, a);
+    else hipLaunchKernelGGL(k_observables<double>, dim3(n_tiles), dim3(lanes), 0, s, a);
     if (a.part) hipLaunchKernelGGL(k_obs_sum, dim3(n_configs), dim3(64), 0, s, a);
     return hipGetLastError();
 }
@@ -3309,7 +3318,8 @@ hipError_t launch_segmented(const SegArgs &a, int fp32, int tw, int lpb, size_t 
 hipError_t launch_hist(const HistArgs &a, hipStream_t s)
 {
     const size_t words = a.gnb <= HIST_WORDS ? std::min<uint64_t>((uint64_t)a.gns * a.gnb, HIST_WORDS) : 0;
-    hipLaunchKernelGGL(k_hist, dim3(a.n_chains * a.parts), dim3(HIST_T), words * sizeof(uint32_t), s, a);
+    const uint32_t lanes = lanes_within((uint64_t)a.n_chains * a.parts, HIST_T, HIST_TILE) >= HIST_T ? HIST_T : HIST_TILE;
+    hipLaunchKernelGGL(k_hist, dim3(a.n_chains * a.parts), dim3(lanes), words * sizeof(uint32_t), s, a);
     return hipGetLastError();
 }
 

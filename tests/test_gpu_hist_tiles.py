@@ -46,3 +46,20 @@ def test_tiled_histograms_equal_oracle(gpu, oracle, boundary, spec):
         assert np.array_equal(x, xs[c]) and np.array_equal(rho[c], want_r), c
         if hs["gns"]:
             assert np.array_equal(g[c], want_g), c
+
+
+def test_many_chains_beside_a_long_one(gpu):
+    """A launch of 64 workgroups a chain whose lanes would pass 2^32 at 1024 a
+    workgroup: every particle is counted all the same."""
+    n = 66000
+    chains = [Chain(N=17000 if c == 1000 else 2, L0=40000.0 if c == 1000 else 40.0, boundary=nat.WALLS, seed=5,
+                    chain_id=c, **lj()) for c in range(n)]
+    print(f"[gpu] histograms of {n} chains", flush=True)
+    with Engine(chains, form="batched_fp64", sample_capacity=1) as e:
+        e.hist_configure(1, rhonb=2, rbw=50000.0, gns=1, gsw=50000.0, gnb=2, gbw=50000.0)
+        e.run(1)
+        rho, g, ns = e.hist_read()
+    assert ns == 1
+    N = np.array([ch.N for ch in chains], dtype=np.uint64)
+    assert np.array_equal(rho.sum(1), N)
+    assert np.array_equal(g.sum((1, 2)), N * (N - np.uint64(1)))
