@@ -103,8 +103,9 @@ typedef struct jmm_engine_opts {
                                  synchronising every (block length - window) phases; a
                                  chain that cannot be split runs from HBM */
     uint32_t seg_lanes;       /* split chains: lanes per block, 1 or 2 (two lanes share each
-                                 trial, one per side, and its box-length sums; 0 = 2 in
-                                 the FP32 form, 1 in the FP64 form); results are the
+                                 trial, one per side, and its box-length sums; 0 = chosen
+                                 by the engine: 2 in the FP32 form where it is faster and
+                                 every segment is resident, else 1); results are the
                                  same bits either way */
     uint32_t sample_virial;   /* 1: after every sweep each chain's virial W = sum -d phi'(d)
                                  and hypervirial sum -d W'(d) are computed (FP64) and kept

@@ -299,6 +299,24 @@ static bool coop_gains(const DevChain &c)
     return c.w >= 2 && (c.B <= 128 || c.w == 2);
 }
 
+// Lanes per block of split chains when the caller leaves them to the engine:
+// two in the FP32 form, except in segments of more than 128 blocks (512-lane
+// workgroups) whose blocks are too short for the two lanes to share the
+// box-length sums (HALF_MIN).  us per sweep, one lane -> two, 1 chain of four
+// segments, windows of 1 (hard rods) / 6 (LJ) / 20 (Yukawa) partners:
+//   64 blocks of 22:   36.3 -> 35.5   52.8 -> 48.0   125.3 -> 115.1
+//   64 blocks of 64:   79.0 -> 68.4  122.1 -> 95.4   264.6 -> 189.5
+//   256 blocks of 22:  42.1 -> 44.4   58.2 -> 60.4   131.4 -> 140.3
+//   256 blocks of 39:  61.1 -> 64.8   88.0 -> 91.2   181.8 -> 196.4
+//   256 blocks of 40:  61.1 -> 60.1   89.6 -> 82.5   184.8 -> 163.2
+//   256 blocks of 64:  87.5 -> 85.8  131.9 -> 120.6  278.5 -> 243.1
+// (20 sigma Yukawa, 40 partners, 256 blocks of 64: 461 -> 380; 40 chains: the
+// same order everywhere).  FP64 walks take one partner at a time: one lane.
+static int seg_lanes_for(int fp32, uint32_t blocks, uint32_t longest_block)
+{
+    return fp32 && (blocks <= 128 || longest_block >= HALF_MIN) ? 2 : 1;
+}
+
 struct jmm_engine {
     int n = 0, form = 0, device = 0, T = 256;
     hipStream_t stream = nullptr;
@@ -951,7 +969,8 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
     // segmented chains: one launch, one workgroup per segment, all resident
     {
         std::vector<DevSeg> segv;
-        uint32_t wgmax = 1, bsmax = 1;
+        uint32_t wgmax = 1, bsmax = 1, seg_smax = 0;
+        uint64_t seg_cost = 0;
         size_t img = 0;
         for (int k = 0; k < n_chains; ++k) {
             const uint32_t S = segS[order[k]];
@@ -970,24 +989,36 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
             wgmax = std::max(wgmax, d.wg);
             bsmax = std::max(bsmax, d.B / S);
             img = std::max(img, 2 * (size_t)d.wg + (size_t)(d.B / S) * d.Sp);
+            // the chain that ends last
+            if (chain_cost(d) >= seg_cost) {
+                seg_cost = chain_cost(d);
+                seg_smax = d.smax;
+            }
         }
         if (!segv.empty()) {
             const int fp32 = e->form == JMM_FORM_BATCHED_FP32;
             if (o.seg_lanes > 2) return bail(fail(JMM_EINVAL, "jmm_create: seg_lanes must be 0, 1 or 2"));
-            e->seg_lpb = o.seg_lanes ? (int)o.seg_lanes : (fp32 ? 2 : 1);
-            e->seg_tw = e->seg_lpb * bsmax > 256 ? 512 : 256;
-            for (int c = 0; c < n_chains; ++c)
-                if (segS[c]) e->layout[c].lanes = (uint32_t)e->seg_lpb;
             e->n_segs = (uint32_t)segv.size();
             e->seg_wgmax = wgmax;
             e->seg_lds_bytes = img * sizeof(double);
-            const void *fn = segmented_kernel(fp32, e->seg_tw, e->seg_lpb);
-            if (int rc = set_lds_attr(fn, e->seg_lds_bytes)) return bail(rc);
-            int occ = 0;
-            CREATE_CHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, e->seg_tw, e->seg_lds_bytes));
-            if ((uint64_t)occ * (uint64_t)n_cu < e->n_segs)
-                return bail(fail(JMM_EINVAL, "jmm_create: split chains need %u workgroups resident at once, "
-                                             "the device holds %d", e->n_segs, occ * n_cu));
+            // all segments resident at once; the engine's own choice of two
+            // lanes (workgroups of twice the lanes, so fewer of them per CU)
+            // gives way to one where they are not
+            e->seg_lpb = o.seg_lanes ? (int)o.seg_lanes : seg_lanes_for(fp32, bsmax, seg_smax);
+            for (;;) {
+                e->seg_tw = e->seg_lpb * bsmax > 256 ? 512 : 256;
+                const void *fn = segmented_kernel(fp32, e->seg_tw, e->seg_lpb);
+                if (int rc = set_lds_attr(fn, e->seg_lds_bytes)) return bail(rc);
+                int occ = 0;
+                CREATE_CHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, e->seg_tw, e->seg_lds_bytes));
+                if ((uint64_t)occ * (uint64_t)n_cu >= e->n_segs) break;
+                if (o.seg_lanes || e->seg_lpb == 1)
+                    return bail(fail(JMM_EINVAL, "jmm_create: split chains need %u workgroups resident at once, "
+                                                 "the device holds %d", e->n_segs, occ * n_cu));
+                e->seg_lpb = 1;
+            }
+            for (int c = 0; c < n_chains; ++c)
+                if (segS[c]) e->layout[c].lanes = (uint32_t)e->seg_lpb;
             if (int rc = dalloc(&e->d_segs, segv.size())) return bail(rc);
             CREATE_CHK(hipMemcpy(e->d_segs, segv.data(), sizeof(DevSeg) * segv.size(), hipMemcpyHostToDevice));
             if (int rc = dalloc(&e->d_pub_head, (size_t)e->n_segs * wgmax)) return bail(rc);

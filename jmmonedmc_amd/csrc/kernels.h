@@ -161,6 +161,13 @@ struct HistArgs {
 }  // namespace jmm
 
 namespace jmm {
+// Where a block's box-length sums are cut in two: sums over the block
+// positions [0, h) and [h, size) are formed apart and added, so that two lanes
+// can share a block (the split kernel) and one lane gives the same bits.
+// Short blocks are not cut: the second walk would cost more than half of one
+// (the 20 sigma Yukawa chains, which the cut is for, have blocks of at least 41).
+constexpr uint32_t HALF_MIN = 40;
+
 hipError_t launch_begin(Ctrl *c, uint32_t n, hipStream_t s);
 // waves: per SIMD, 2 or (T = 256 in LDS) 3
 const void *batched_kernel(int fp32, int T, int gx, int waves);

@@ -945,13 +945,6 @@ __device__ __forceinline__ bool trial_lds(const LdsChain &c, const Pot &q, doubl
     return go && (dE <= 0.0 || (double)bf > u);
 }
 
-// Where a block's box-length sums are cut in two: sums over the block
-// positions [0, h) and [h, size) are formed apart and added, so that two lanes
-// can share a block (the split kernel) and one lane gives the same bits.
-// Short blocks are not cut: the second walk would cost more than half of one
-// (the 20 sigma Yukawa chains, which the cut is for, have blocks of at least 41).
-constexpr uint32_t HALF_MIN = 40;
-
 __device__ __forceinline__ uint32_t half_of(uint32_t size)
 {
     return size >= HALF_MIN ? (size + 1) / 2 : size;
