@@ -2126,6 +2126,16 @@ __device__ __forceinline__ uint64_t seg_pidx(uint32_t j, uint32_t par, uint32_t 
     return (((uint64_t)j * 2 + par) * SEG_FIELDS + f) * SEG_WAVES + wv;
 }
 
+// The sums' scratch of a segment's workgroup.  The image of a segment leaves
+// 512 bytes of the LDS (the splitting threshold); one for the four potentials.
+template <int TW>
+struct SegScratch {
+    double rd[(TW / 64) * 3];
+    double tot[SEG_FIELDS];
+    uint32_t ri[(TW / 64) * 4];
+};
+static_assert(sizeof(SegScratch<256>) <= 512 && sizeof(SegScratch<512>) <= 512, "LDS left to a segment's image");
+
 // One segment of a chain: blocks s*Bs .. s*Bs+Bs-1, one lane each, in LDS
 // with halos of wg positions on either side that hold the neighbouring
 // segments' boundary particles (periodic images at the chain's ends, as the
@@ -2156,7 +2166,7 @@ __device__ __forceinline__ uint64_t seg_pidx(uint32_t j, uint32_t par, uint32_t 
 // parity: a segment is at most one all-segment point ahead of another.
 template <typename Real, int KIND, int TW, int LPB>
 __device__ __forceinline__ void run_segment(const SegArgs &g, const DevSeg &sg, double *smem,
-                            BatchedScratch<TW> &sc, uint32_t soff)
+                            SegScratch<TW> &sc, uint32_t soff)
 {
     const SweepArgs &a = g.a;
     const uint32_t tid = threadIdx.x;
@@ -2269,7 +2279,7 @@ __device__ __forceinline__ void run_segment(const SegArgs &g, const DevSeg &sg, 
     // over B = S*Bs lanes: pairwise trees within 64-lane groups, the group
     // totals then added in sequence from zero (no sequence when B <= 64).
     // Every segment reads the same values in the same order: the same bits.
-    __shared__ double tot[SEG_FIELDS];
+    double *tot = sc.tot;
     auto gather = [&](uint32_t par, uint32_t f) {
         if (tid < 64) {
             double acc = 0.0;
@@ -2540,7 +2550,7 @@ __global__ void __launch_bounds__(TW) __attribute__((amdgpu_waves_per_eu(1)))
 k_sweep_seg(SegArgs g)
 {
     extern __shared__ double smem[];
-    __shared__ BatchedScratch<TW> sc;
+    __shared__ SegScratch<TW> sc;
     const uint32_t soff = g.a.ctrl->sample_off;
     const DevSeg sg = g.segs[blockIdx.x];
     switch (g.a.chains[sg.chain].kind) {

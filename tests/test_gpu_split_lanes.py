@@ -67,3 +67,18 @@ def test_choice_by_segment_and_block_length(gpu, form):
                 l = e.layout(0)
             assert l["mode"] == "split" and l["B"] // l["segments"] == blocks, (N, bcap, l)
             assert l["lanes"] == (lanes if form == "batched_fp32" else 1), (N, bcap, l)
+
+
+@pytest.mark.parametrize("form", ["batched_fp32", "batched_fp64"])
+@pytest.mark.parametrize("lanes", [0, 1, 2])
+def test_largest_segment_image(gpu, form, lanes):
+    """Segments whose images leave just the 512 bytes of LDS that the split
+    threshold sets aside (8 blocks of 5099, 2 segments of 20,408 doubles of the
+    20,416): accepted, and equal to the chain in more segments."""
+    print(f"[gpu] split lanes: largest image {form} {lanes}", flush=True)
+    ch = npt(8 * 5099, 0, 8)
+    lay, smp, x = go([ch], lanes, form=form)
+    assert lay[0]["mode"] == "split" and lay[0]["segments"] == 2 and lay[0]["lds_bytes"] == 8 * 20408
+    lay4, smp4, x4 = go([ch], lanes, seg_lds=90000, form=form)
+    assert lay4[0]["segments"] == 4
+    assert np.array_equal(smp, smp4) and np.array_equal(x[0], x4[0])
