@@ -113,6 +113,7 @@ struct ObsArgs {
     const uint64_t *goff;    // engine form, nullable: gradient offset of each chain (else x_off)
     uint32_t tile, parts;    // particles per workgroup; standalone form: workgroups per configuration
     uint32_t standalone;
+    uint32_t group0;         // first workgroup of this launch
 };
 
 // A chain too large for one workgroup's LDS is split into S segments of Bs
@@ -185,8 +186,7 @@ const void *coop_kernel(int fp32);
 hipError_t launch_coop(const SweepArgs &a, int fp32, uint32_t grid, uint32_t threads, size_t lds, hipStream_t s);
 const void *plain_kernel(int gx);
 hipError_t launch_plain(const SweepArgs &a, int gx, uint32_t grid, size_t lds, hipStream_t s);
-hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads,
-                              hipStream_t s);
+hipError_t launch_observables(ObsArgs a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads, hipStream_t s);
 // Samples in the caller's layout (jmm_sample): out[ext[k] * n_sweeps + s]
 // from the engine's [sweep][chain] arrays.
 struct SampleRec {

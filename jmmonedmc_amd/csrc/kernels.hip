@@ -2801,6 +2801,10 @@ __device__ __forceinline__ void pair_obs_f(const Pot &q, double rsig, double d, 
     f = (double)o[1] / d;
 }
 
+// Waves of a tile.
+constexpr uint32_t OBS_WAVES = OBS_TILE / 64;
+static_assert(OBS_ONE <= 2 * OBS_TILE, "k_obs_sum adds two tiles as v0 + v1");
+
 // LDS of the observables kernel: the waves' sums, forces handed to the next
 // wave, and the edge's forces by wave.
 struct ObsScratch {
@@ -2826,6 +2830,12 @@ struct ObsScratch {
 // index distance (left to the first wave they cost as much as both walks did:
 // it sits on the same SIMD in every workgroup).  The walk is uniform over the
 // wave with the next position loaded ahead.
+// A configuration's sums and gradients are the same bits whatever the workgroup
+// (engines take it from the longest chain): waves are added up per OBS_TILE
+// particles, then the tiles as k_obs_sum does; a workgroup of two tiles
+// evaluates the pairs across their boundary again as two workgroups do; and an
+// edge's partners are summed in as many strides as the tile's particles have
+// waves, whatever the workgroup has.
 // The kernel, FP32: 64 Yukawa configurations of 65,536 314 us with both sides
 // walked, 244 with each pair once, 225 with the divisions of pair_obs_f and
 // tiles of 512; 1024 LJ chains of 1024 28 and 22 us.
@@ -2834,7 +2844,8 @@ __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, dou
                                         uint32_t p1, double *out, double *grad, ObsScratch &sm)
 {
     double *red = sm.red, *next = sm.next, *edge = sm.edge;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, waves = blockDim.x >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, waves = blockDim.x >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const Pot q = ch.pot;
     const uint32_t N = ch.N;
     // a compressed configuration (sc < 1) may hold gaps below the hard core:
@@ -2915,13 +2926,16 @@ __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, dou
             return s;
         };
         next[tid] = gn;
-        edge[tid] = t0 + lane < p1 ? left(t0 + lane, lane + 1 + wave, waves) : 0.0;
+        const uint32_t first = wave / OBS_WAVES * OBS_WAVES, m = t0 + first * 64 + lane;
+        // waves of the tile that hold particles (no more than the workgroup's)
+        const uint32_t strides = min(OBS_WAVES, (p1 - min(p1, t0 + first * 64) + 63) / 64);
+        edge[tid] = wave - first < strides && m < p1 ? left(m, lane + 1 + wave - first, strides) : 0.0;
         __syncthreads();
-        if (wave) {
+        if (wave != first) {
             gl += next[tid - 64];
             if (i < p1) gl += left(i, 65, 1);
         } else {
-            for (uint32_t v = 0; v < waves; ++v) gl += edge[v * 64 + lane];
+            for (uint32_t v = 0; v < strides; ++v) gl += edge[tid + v * 64];
         }
         if (i < p1) grad[i] = g - gl;
         __syncthreads();
@@ -2931,10 +2945,17 @@ __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, dou
     if ((tid & 63) == 0)
         for (int m = 0; m < 6; ++m) red[(tid >> 6) * 6 + m] = acc[m];
     __syncthreads();
-    if (tid < 6) {
+    // a tile's waves in order, then the tiles: a lane per field and tile
+    if (tid < 12) {
+        const uint32_t half = tid / 6, field = tid - half * 6;
         double v = 0.0;
-        for (uint32_t wv = 0; wv < (blockDim.x >> 6); ++wv) v += red[wv * 6 + tid];
-        out[tid] = v;
+#pragma unroll
+        for (uint32_t wv = 0; wv < OBS_WAVES; ++wv) {
+            const uint32_t from = half * OBS_WAVES + wv;
+            v += from < waves ? red[from * 6 + field] : 0.0;
+        }
+        const double second = __shfl(v, (int)tid + 6);
+        if (tid < 6) out[tid] = v + second;
     }
 }
 
@@ -2948,15 +2969,16 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(sizeo
 k_observables(ObsArgs a)
 {
     __shared__ ObsScratch sm;  // one for the four potentials
+    const uint32_t group = a.group0 + blockIdx.x;
     uint32_t c, p0 = 0, part = 0;
     if (a.standalone) {
-        c = blockIdx.x / a.parts;
-        part = blockIdx.x % a.parts;
+        c = group / a.parts;
+        part = group % a.parts;
     } else if (a.tiles) {
-        c = a.tiles[blockIdx.x].chain;
-        part = a.tiles[blockIdx.x].part;
+        c = a.tiles[group].chain;
+        part = a.tiles[group].part;
     } else {
-        c = blockIdx.x;
+        c = group;
     }
     const DevChain &ch = a.standalone ? a.one : a.chains[c];
     const uint32_t N = ch.N;
@@ -2978,7 +3000,7 @@ k_observables(ObsArgs a)
         }
         grad = a.grad ? a.grad + (a.goff ? a.goff[c] : ch.x_off) : nullptr;
     }
-    if (a.part) out = a.part + (uint64_t)blockIdx.x * 6;
+    if (a.part) out = a.part + (uint64_t)group * 6;
     else out = a.obs + (uint64_t)(a.row ? a.row[c] : c) * 6;
     switch (ch.kind) {
     case POT_LJ: run_obs<Real, POT_LJ>(ch, X, L, sc, p0, p1, out, grad, sm); break;
@@ -3278,12 +3300,17 @@ static uint32_t lanes_within(uint64_t groups, uint32_t want, uint32_t least)
     return (uint32_t)std::max<uint64_t>(least, std::min<uint64_t>(want, most));
 }
 
-hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads,
-                              hipStream_t s)
+hipError_t launch_observables(ObsArgs a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads, hipStream_t s)
 {
-    const uint32_t lanes = lanes_within(n_tiles, (uint32_t)threads, 64);
-    if (fp32) hipLaunchKernelGGL(k_observables<float>, dim3(n_tiles), dim3(lanes), 0, s, a);
-    else hipLaunchKernelGGL(k_observables<double>, dim3(n_tiles), dim3(lanes), 0, s, a);
+    // a launch holds fewer than 2^32 lanes
+    const uint32_t most = 0xffffffffu / (uint32_t)threads;
+    for (uint32_t done = 0; done < n_tiles;) {
+        const uint32_t n = std::min(n_tiles - done, most);
+        a.group0 = done;
+        if (fp32) hipLaunchKernelGGL(k_observables<float>, dim3(n), dim3(threads), 0, s, a);
+        else hipLaunchKernelGGL(k_observables<double>, dim3(n), dim3(threads), 0, s, a);
+        done += n;
+    }
     if (a.part) hipLaunchKernelGGL(k_obs_sum, dim3(n_configs), dim3(64), 0, s, a);
     return hipGetLastError();
 }
