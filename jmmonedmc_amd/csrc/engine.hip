@@ -345,7 +345,7 @@ struct jmm_engine {
     uint8_t *d_log = nullptr;
     double *d_obs = nullptr, *d_grad = nullptr, *d_Lnew = nullptr;
     // observables kernel: tiles of long chains, their partial sums
-    ObsTile *d_tiles = nullptr;
+    Tile *d_tiles = nullptr;
     uint32_t *d_first = nullptr;
     double *d_obs_part = nullptr;
     uint32_t obs_tiles = 0;
@@ -376,6 +376,8 @@ struct jmm_engine {
     uint32_t hist_every = 0;
     jmm_hist_spec hs{};
     unsigned long long *d_rho = nullptr, *d_g = nullptr;
+    Tile *d_hist_tiles = nullptr;
+    uint32_t hist_tiles = 0;
     uint64_t hist_samples = 0;
 };
 
@@ -633,6 +635,7 @@ int jmm_destroy(jmm_engine *e)
     (void)hipFree(e->d_obs_part);
     (void)hipFree(e->d_rho);
     (void)hipFree(e->d_g);
+    (void)hipFree(e->d_hist_tiles);
     (void)hipFree(e->d_packed);
     (void)hipHostFree(e->h_stage);
     (void)hipFree(e->d_ext);
@@ -1068,15 +1071,11 @@ static int launch_hist_sample(jmm_engine *e)
     h.rbw = e->hs.rbw;
     h.gsw = e->hs.gsw;
     h.gbw = e->hs.gbw;
-    h.n_chains = (uint32_t)e->n;
+    h.tiles = e->d_hist_tiles;
+    h.n_tiles = e->hist_tiles;
     h.rhonb = e->hs.rhonb;
     h.gns = e->hs.gns;
     h.gnb = e->hs.gnb;
-    uint64_t nmax = 1;
-    for (const auto &c : e->hch) nmax = std::max<uint64_t>(nmax, c.N);
-    // a workgroup per tile; of engines with many chains as long as the parts of
-    // the longest (the others' return at once) stay within some ten rounds
-    h.parts = (uint32_t)std::min<uint64_t>((nmax + HIST_TILE - 1) / HIST_TILE, std::max<uint64_t>(64, 4096 / e->n));
     HIPCHK(launch_hist(h, e->stream));
     e->hist_samples++;
     return 0;
@@ -1098,6 +1097,18 @@ int jmm_hist_configure(jmm_engine *e, const jmm_hist_spec *spec, uint32_t every)
     if (h.rhonb == 0 || !(h.rbw > 0.0) || (h.gns && (!(h.gsw > 0.0) || h.gnb == 0 || !(h.gbw > 0.0))))
         return fail(JMM_EINVAL, "jmm_hist_configure: bin counts and widths must be positive");
     const uint64_t nr = (uint64_t)e->n * h.rhonb, ng = (uint64_t)e->n * h.gns * h.gnb;
+    if (!e->hist_tiles) {
+        std::vector<Tile> tiles;
+        for (uint32_t k = 0; k < (uint32_t)e->n; ++k) {
+            const uint32_t N = e->hch[k].N, P = hist_tile(N);
+            for (uint32_t p = 0; p < (N + P - 1) / P; ++p) tiles.push_back({k, p});
+        }
+        // (an attempt that failed half-way kept the buffer)
+        if (!e->d_hist_tiles)
+            if (int rc = dalloc(&e->d_hist_tiles, tiles.size())) return rc;
+        HIPCHK(hipMemcpy(e->d_hist_tiles, tiles.data(), sizeof(Tile) * tiles.size(), hipMemcpyHostToDevice));
+        e->hist_tiles = (uint32_t)tiles.size();
+    }
     if (int rc = dalloc(&e->d_rho, nr)) return rc;
     if (ng)
         if (int rc = dalloc(&e->d_g, ng)) return rc;
@@ -1581,7 +1592,7 @@ static int ensure_obs(jmm_engine *e)
     uint32_t nmax = 1;
     for (const auto &c : e->hch) nmax = std::max(nmax, c.N);
     if (nmax > OBS_ONE && !e->obs_tiles) {
-        std::vector<ObsTile> tiles;
+        std::vector<Tile> tiles;
         std::vector<uint32_t> first(1, 0u);
         for (uint32_t k = 0; k < (uint32_t)e->n; ++k) {
             for (uint32_t p = 0; p * OBS_TILE < e->hch[k].N; ++p) tiles.push_back({k, p});
@@ -1594,7 +1605,7 @@ static int ensure_obs(jmm_engine *e)
             if (int rc = dalloc(&e->d_first, first.size())) return rc;
         if (!e->d_obs_part)
             if (int rc = dalloc(&e->d_obs_part, tiles.size() * 6)) return rc;
-        HIPCHK(hipMemcpy(e->d_tiles, tiles.data(), sizeof(ObsTile) * tiles.size(), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(e->d_tiles, tiles.data(), sizeof(Tile) * tiles.size(), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(e->d_first, first.data(), sizeof(uint32_t) * first.size(), hipMemcpyHostToDevice));
         e->obs_tiles = (uint32_t)tiles.size();
         e->obs_threads = (int)OBS_TILE;

@@ -83,8 +83,8 @@ struct SweepArgs {
     uint32_t n_items, n_sweeps, n_chains, cap;
 };
 
-// A tile of a configuration: particles [part * OBS_TILE, (part + 1) * OBS_TILE).
-struct ObsTile {
+// A tile of a chain's configuration: its part-th run of a tile's particles.
+struct Tile {
     uint32_t chain, part;
 };
 
@@ -103,7 +103,7 @@ struct ObsArgs {
     DevChain one;            // standalone form
     const double *x;
     const double *L;         // standalone form
-    const ObsTile *tiles;    // engine form, nullable: tiles of all chains in chain order
+    const Tile *tiles;       // engine form, nullable: tiles of all chains in chain order
     const uint32_t *first;   // engine form with tiles: [n + 1], first tile of each chain
     const double *Lnew;      // engine form, nullable: evaluate at x * Lnew/L, length Lnew
     double *part;            // nullable: [tile][6] partial sums, for k_obs_sum
@@ -142,21 +142,26 @@ struct SegArgs {
     uint32_t wgmax, n_segs;
 };
 
-// rho(x) and g(x) histograms of every chain's current configuration.
-// Histogram kernel: lanes of a workgroup (HIST_TILE of them where a launch's
-// limit asks for it), particles of a tile, 32-bit counters
-// in LDS (64 KB: two workgroups per CU), and the longest chain whose tiles
-// cannot overflow them (HIST_TILE particles, N - 1 partners, both members).
+// Histogram kernel: lanes of a workgroup (HIST_TILE of them without g(x), which
+// has one count a particle), particles of a tile (short chains: fewer, with more
+// lanes a particle), 32-bit counters in LDS (64 KB: two workgroups per CU), and
+// the longest chain whose tiles cannot overflow them (HIST_TILE particles, N - 1
+// partners, both members).
 constexpr uint32_t HIST_T = 1024, HIST_TILE = 256, HIST_WORDS = 16384, HIST_N_LDS = 1u << 22;
 
+__host__ __device__ inline uint32_t hist_tile(uint32_t N) { return N <= 64 ? 64u : N <= 128 ? 128u : HIST_TILE; }
+
+// rho(x) and g(x) histograms of every chain's current configuration.
 struct HistArgs {
     const DevChain *chains;
     const DevState *states;
     const double *x;
+    const Tile *tiles;        // of all chains
     unsigned long long *rho;  // [chain][rhonb]
     unsigned long long *g;    // [chain][gns][gnb]
     double rbw, gsw, gbw;
-    uint32_t n_chains, rhonb, gns, gnb, parts;
+    uint32_t n_tiles, rhonb, gns, gnb;
+    uint32_t group0;          // first workgroup of this launch
 };
 
 }  // namespace jmm
@@ -186,7 +191,8 @@ const void *coop_kernel(int fp32);
 hipError_t launch_coop(const SweepArgs &a, int fp32, uint32_t grid, uint32_t threads, size_t lds, hipStream_t s);
 const void *plain_kernel(int gx);
 hipError_t launch_plain(const SweepArgs &a, int gx, uint32_t grid, size_t lds, hipStream_t s);
-hipError_t launch_observables(ObsArgs a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads, hipStream_t s);
+hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads,
+                              hipStream_t s);
 // Samples in the caller's layout (jmm_sample): out[ext[k] * n_sweeps + s]
 // from the engine's [sweep][chain] arrays.
 struct SampleRec {

@@ -3136,17 +3136,17 @@ __device__ __forceinline__ int64_t bin_of(double x, double width, uint32_t nb)
 // larger chains count in memory.
 // 32 chains of 2000, 10 segments of 1000 bins: 95 us a sample with a particle
 // per lane and atomics to memory, 15.5 us so.
-// Grid: chains x parts, the parts of a chain stride over its tiles.
+// Grid: a workgroup per tile of every chain (workgroups for each chain's share
+// of the longest one's tiles, most of them empty, cost more than the counting:
+// 512 chains of 32 beside 4 of 60,000, rho alone 7.1 us against 94).
 __global__ void __launch_bounds__(HIST_T) k_hist(HistArgs a)
 {
     extern __shared__ uint32_t hw[];
-    const uint32_t c = blockIdx.x / a.parts, part = blockIdx.x % a.parts, tid = threadIdx.x;
+    const Tile at = a.tiles[a.group0 + blockIdx.x];
+    const uint32_t c = at.chain, tid = threadIdx.x;
     const DevChain &ch = a.chains[c];
     const uint32_t N = ch.N;
-    // particles of a tile (short chains: more lanes per particle)
-    const uint32_t P = N <= 64 ? 64u : N <= 128 ? 128u : HIST_TILE, K = blockDim.x / P;
-    const uint32_t tiles = (N + P - 1) / P;
-    if (part >= tiles) return;
+    const uint32_t P = hist_tile(N), K = blockDim.x / P;
     const bool per = (ch.flags & F_PERIODIC) != 0;
     const double L = a.states[c].L;
     const double *X = a.x + ch.x_off;
@@ -3154,60 +3154,57 @@ __global__ void __launch_bounds__(HIST_T) k_hist(HistArgs a)
     unsigned long long *rho = a.rho + (uint64_t)c * a.rhonb;
     unsigned long long *g = a.g + (uint64_t)c * a.gns * a.gnb;
     const uint32_t kl = tid / P;
-    for (uint32_t tile = part; tile < tiles; tile += a.parts) {
-        const uint32_t p0 = tile * P, i = p0 + tid % P;
-        // window of segments counted in LDS: from the first particle's to the
-        // last one's farthest partner's, where they lie in that order
-        uint32_t s0 = 0, W = 0;
-        if (N <= HIST_N_LDS && a.gns && a.gnb && a.gnb <= HIST_WORDS) {
-            const double f0 = fold(X[p0], L, per), f1 = fold(X[min(p0 + P, N) - 1], L, per) + gmax;
-            const int64_t top = (int64_t)a.gns - 1;
-            const int64_t b0 = max((int64_t)0, min(top, bin_of(f0, a.gsw, a.gns)));
-            const int64_t b1 = max(b0, min(top, bin_of(f1, a.gsw, a.gns)));
-            s0 = (uint32_t)b0;
-            W = (uint32_t)min((int64_t)(HIST_WORDS / a.gnb), (f1 < f0 ? top : b1) - b0 + 1);
-        }
-        const uint32_t words = W * a.gnb;
-        for (uint32_t m = tid; m < words; m += blockDim.x) hw[m] = 0;
-        __syncthreads();
-        if (i < N) {
-            const double xi = X[i];
-            const double fi = fold(xi, L, per);
-            if (kl == 0) {
-                const int64_t rb = bin_of(fi, a.rbw, a.rhonb);
-                if (rb >= 0 && rb < (int64_t)a.rhonb) atomicAdd(&rho[rb], 1ull);
-            }
-            const int64_t si = bin_of(fi, a.gsw, a.gns);
-            const uint32_t kmax = a.gns && a.gnb ? N : 0;
-            for (uint32_t k = 1 + kl; k < kmax; k += K) {
-                const uint32_t j0 = i + k;
-                double d, xj;
-                if (j0 < N) {
-                    xj = X[j0];
-                    d = xj - xi;
-                } else {
-                    if (!per) break;
-                    xj = X[j0 - N];
-                    d = (xj + L) - xi;
-                }
-                if (!(d < gmax) || (per && !(d < L / 2.0))) break;
-                const int64_t gb = (int64_t)floor(d / a.gbw);
-                if (gb < 0 || gb >= (int64_t)a.gnb) continue;
-                const int64_t sj = bin_of(fold(xj, L, per), a.gsw, a.gns);
-                const uint64_t ri = (uint64_t)(si - (int64_t)s0), rj = (uint64_t)(sj - (int64_t)s0);
-                if (ri < W) atomicAdd(&hw[(uint32_t)ri * a.gnb + (uint32_t)gb], si == sj ? 2u : 1u);
-                else if (si >= 0 && si < (int64_t)a.gns)
-                    atomicAdd(&g[(uint64_t)si * a.gnb + gb], si == sj ? 2ull : 1ull);
-                if (si == sj) continue;
-                if (rj < W) atomicAdd(&hw[(uint32_t)rj * a.gnb + (uint32_t)gb], 1u);
-                else if (sj >= 0 && sj < (int64_t)a.gns) atomicAdd(&g[(uint64_t)sj * a.gnb + gb], 1ull);
-            }
-        }
-        __syncthreads();
-        for (uint32_t m = tid; m < words; m += blockDim.x)
-            if (const uint32_t v = hw[m]) atomicAdd(&g[(uint64_t)s0 * a.gnb + m], (unsigned long long)v);
-        __syncthreads();
+    const uint32_t p0 = at.part * P, i = p0 + tid % P;
+    // window of segments counted in LDS: from the first particle's to the
+    // last one's farthest partner's, where they lie in that order
+    uint32_t s0 = 0, W = 0;
+    if (N <= HIST_N_LDS && a.gns && a.gnb && a.gnb <= HIST_WORDS) {
+        const double f0 = fold(X[p0], L, per), f1 = fold(X[min(p0 + P, N) - 1], L, per) + gmax;
+        const int64_t top = (int64_t)a.gns - 1;
+        const int64_t b0 = max((int64_t)0, min(top, bin_of(f0, a.gsw, a.gns)));
+        const int64_t b1 = max(b0, min(top, bin_of(f1, a.gsw, a.gns)));
+        s0 = (uint32_t)b0;
+        W = (uint32_t)min((int64_t)(HIST_WORDS / a.gnb), (f1 < f0 ? top : b1) - b0 + 1);
     }
+    const uint32_t words = W * a.gnb;
+    for (uint32_t m = tid; m < words; m += blockDim.x) hw[m] = 0;
+    __syncthreads();
+    if (i < N) {
+        const double xi = X[i];
+        const double fi = fold(xi, L, per);
+        if (kl == 0) {
+            const int64_t rb = bin_of(fi, a.rbw, a.rhonb);
+            if (rb >= 0 && rb < (int64_t)a.rhonb) atomicAdd(&rho[rb], 1ull);
+        }
+        const int64_t si = bin_of(fi, a.gsw, a.gns);
+        const uint32_t kmax = a.gns && a.gnb ? N : 0;
+        for (uint32_t k = 1 + kl; k < kmax; k += K) {
+            const uint32_t j0 = i + k;
+            double d, xj;
+            if (j0 < N) {
+                xj = X[j0];
+                d = xj - xi;
+            } else {
+                if (!per) break;
+                xj = X[j0 - N];
+                d = (xj + L) - xi;
+            }
+            if (!(d < gmax) || (per && !(d < L / 2.0))) break;
+            const int64_t gb = (int64_t)floor(d / a.gbw);
+            if (gb < 0 || gb >= (int64_t)a.gnb) continue;
+            const int64_t sj = bin_of(fold(xj, L, per), a.gsw, a.gns);
+            const uint64_t ri = (uint64_t)(si - (int64_t)s0), rj = (uint64_t)(sj - (int64_t)s0);
+            if (ri < W) atomicAdd(&hw[(uint32_t)ri * a.gnb + (uint32_t)gb], si == sj ? 2u : 1u);
+            else if (si >= 0 && si < (int64_t)a.gns)
+                atomicAdd(&g[(uint64_t)si * a.gnb + gb], si == sj ? 2ull : 1ull);
+            if (si == sj) continue;
+            if (rj < W) atomicAdd(&hw[(uint32_t)rj * a.gnb + (uint32_t)gb], 1u);
+            else if (sj >= 0 && sj < (int64_t)a.gns) atomicAdd(&g[(uint64_t)sj * a.gnb + gb], 1ull);
+        }
+    }
+    __syncthreads();
+    for (uint32_t m = tid; m < words; m += blockDim.x)
+        if (const uint32_t v = hw[m]) atomicAdd(&g[(uint64_t)s0 * a.gnb + m], (unsigned long long)v);
 }
 
 // Positions of every chain scaled to a new length: x -> x Lnew/L (moveVolume,
@@ -3292,25 +3289,22 @@ hipError_t launch_plain(const SweepArgs &a, int gx, uint32_t grid, size_t lds, h
     return hipGetLastError();
 }
 
-// Lanes of a workgroup: as wanted, or fewer (whole waves, at least `least`)
-// where a launch of so many workgroups would pass its limit of 2^32 lanes.
-static uint32_t lanes_within(uint64_t groups, uint32_t want, uint32_t least)
+// Launches n_groups workgroups in parts that stay below a launch's 2^32 lanes.
+template <typename Args>
+static void launch_groups(void (*kernel)(Args), Args a, uint32_t n_groups, uint32_t lanes, size_t lds, hipStream_t s)
 {
-    const uint64_t most = groups ? 0xffffffffull / groups / 64 * 64 : want;
-    return (uint32_t)std::max<uint64_t>(least, std::min<uint64_t>(want, most));
+    const uint32_t most = 0xffffffffu / lanes;
+    for (a.group0 = 0; a.group0 < n_groups;) {
+        const uint32_t n = std::min(n_groups - a.group0, most);
+        hipLaunchKernelGGL(kernel, dim3(n), dim3(lanes), lds, s, a);
+        a.group0 += n;
+    }
 }
 
-hipError_t launch_observables(ObsArgs a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads, hipStream_t s)
+hipError_t launch_observables(const ObsArgs &a, int fp32, uint32_t n_tiles, uint32_t n_configs, int threads,
+                              hipStream_t s)
 {
-    // a launch holds fewer than 2^32 lanes
-    const uint32_t most = 0xffffffffu / (uint32_t)threads;
-    for (uint32_t done = 0; done < n_tiles;) {
-        const uint32_t n = std::min(n_tiles - done, most);
-        a.group0 = done;
-        if (fp32) hipLaunchKernelGGL(k_observables<float>, dim3(n), dim3(threads), 0, s, a);
-        else hipLaunchKernelGGL(k_observables<double>, dim3(n), dim3(threads), 0, s, a);
-        done += n;
-    }
+    launch_groups(fp32 ? k_observables<float> : k_observables<double>, a, n_tiles, (uint32_t)threads, 0, s);
     if (a.part) hipLaunchKernelGGL(k_obs_sum, dim3(n_configs), dim3(64), 0, s, a);
     return hipGetLastError();
 }
@@ -3348,8 +3342,7 @@ hipError_t launch_segmented(const SegArgs &a, int fp32, int tw, int lpb, size_t 
 hipError_t launch_hist(const HistArgs &a, hipStream_t s)
 {
     const size_t words = a.gnb <= HIST_WORDS ? std::min<uint64_t>((uint64_t)a.gns * a.gnb, HIST_WORDS) : 0;
-    const uint32_t lanes = lanes_within((uint64_t)a.n_chains * a.parts, HIST_T, HIST_TILE) >= HIST_T ? HIST_T : HIST_TILE;
-    hipLaunchKernelGGL(k_hist, dim3(a.n_chains * a.parts), dim3(lanes), words * sizeof(uint32_t), s, a);
+    launch_groups(k_hist, a, a.n_tiles, a.gns && a.gnb ? HIST_T : HIST_TILE, words * sizeof(uint32_t), s);
     return hipGetLastError();
 }
 
