@@ -9,11 +9,13 @@
 #include <cstdio>
 #include <cstddef>
 #include <cstring>
+#include <functional>
 #include <limits>
 #include <memory>
 #include <mutex>
 #include <new>
 #include <numeric>
+#include <queue>
 #include <string>
 #include <vector>
 
@@ -273,13 +275,6 @@ struct Group {
     uint32_t *d_list = nullptr;
 };
 
-// Most waves per CU (of its 32) at which an engine's chains run one per
-// workgroup with several lanes per block: beyond, the extra lanes' work costs
-// more than the latency they save.  us per sweep, one lane -> several, LJ NPT
-// FP32: 1024 chains of 64 (8 waves per CU) 17.9 -> 10.6, 2048 (16) 17.9 -> 26.9;
-// 256 of 250 (8) 17.5 -> 11.2, 512 (16) 17.7 -> 22.0.
-constexpr uint64_t COOP_WAVES = 8;
-
 // LDS that a batched workgroup takes beside its bundle's image: at most 512
 // bytes, and what the allocation is rounded up by.
 constexpr size_t BATCHED_STATIC = 2560;
@@ -297,6 +292,55 @@ static uint64_t chain_cost(const DevChain &c) { return (uint64_t)c.smax * (c.w +
 static bool coop_gains(const DevChain &c)
 {
     return c.w >= 2 && (c.B <= 128 || c.w == 2);
+}
+
+// Whether chains that are launched one per workgroup, in this order, end
+// before they would with one lane per block.  All resident at once (the launch
+// gives every workgroup the lanes and the LDS of the largest chain, so `slots`
+// of them): yes, where the longest gains (coop_gains).  Otherwise the later
+// ones wait for the earlier, while with one lane every chain runs at once: the
+// launch's end is taken from the chains' estimated times, each on the slot that
+// is free first, and compared with the longest chain's on one lane.  The
+// estimates, us per sweep, are fits to LJ and hard-rod chains of 25 to 1000:
+// 0.05 (cost + 100) with several lanes (times 1.04 to 1.5 for 1 to 8 waves at
+// 16 lanes per block, 1.8 at 4, 2.5 at 2), 0.225 (FP64 0.295) (cost + 16) with
+// one.  Measured, one lane -> several, FP32 / FP64 (taken where marked *):
+//   log-uniform 20 to 256, LJ and rods, 300 chains  28.9 -> 11.4* / 37.5 -> 12.7*
+//                                       600         28.5 -> 20.2* / 37.5 -> 22.6*
+//                                      1500         28.6 -> 44.9  / 37.6 -> 50.4
+//   300 of 25 beside one of 300                     26.9 -> 20.9* / 35.4 -> 23.8*
+//   1000 of 25 beside one of 300                    27.0 -> 40.8  / 35.2 -> 45.8
+//   1024 of 64 (all resident)                       18.2 -> 10.1* / 23.4 -> 11.8*
+//   257 of 250 (256 resident)                       18.0 -> 20.3  / 23.5 -> 23.3
+static bool coop_in_time(const std::vector<DevChain> &ch, const std::vector<uint32_t> &order, size_t slots, bool fp32)
+{
+    if (order.size() <= slots) return true;
+    if (!slots) return false;
+    auto several = [&](const DevChain &c) {
+        const double waves = coop_threads(c) / 64, lanes = coop_lanes(c.B);
+        const double f = lanes == 16 ? (fp32 ? 1.0 + 0.04 * waves : 1.05 + 0.055 * waves)
+                       : lanes == 4  ? (fp32 ? 1.75 : 1.85)
+                                     : 2.5;
+        return 0.05 * (double)(chain_cost(c) + 100) * f;
+    };
+    double limit = 0.0, work = 0.0;
+    for (uint32_t c : order) {
+        limit = std::max(limit, 0.95 * (fp32 ? 0.225 : 0.295) * (double)(chain_cost(ch[c]) + 16));
+        work += several(ch[c]);
+    }
+    if (work > limit * (double)slots) return false;
+    std::priority_queue<double, std::vector<double>, std::greater<double>> ends;
+    for (uint32_t c : order) {
+        double start = 0.0;
+        if (ends.size() == slots) {
+            start = ends.top();
+            ends.pop();
+        }
+        const double end = start + several(ch[c]);
+        if (end > limit) return false;
+        ends.push(end);
+    }
+    return true;
 }
 
 // Lanes per block of split chains when the caller leaves them to the engine:
@@ -742,20 +786,33 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
 
     // Engines with too few chains to fill the GPU give each a workgroup with
     // several lanes per block (k_sweep_coop), where every chain that is not
-    // split is short-ranged enough for it, the longest gains by it (coop_gains;
-    // the others end before it) and all of them are resident at COOP_WAVES
-    // waves per CU.
+    // split is short-ranged enough for it, the longest gains by it (coop_gains)
+    // and the launch ends in time (coop_in_time).
+    const bool fp32 = e->form == JMM_FORM_BATCHED_FP32;
     bool coop = e->form != JMM_FORM_PLAIN_FP64 && o.block_lanes != 1;
-    uint64_t coop_waves = 0;
-    int longest = -1;
+    std::vector<uint32_t> coop_order;  // the longest first: they end last
+    uint32_t coop_threads_max = 0;
+    size_t coop_lds_max = 0;
     for (int c = 0; c < n_chains && coop; ++c) {
         if (segS[c]) continue;
         if (ch[c].w > COOP_W || ch[c].B > COOP_B || coop_lds(ch[c]) > (size_t)lds_max - 1024) coop = false;
-        coop_waves += coop_threads(ch[c]) / 64;
-        if (longest < 0 || chain_cost(ch[c]) > chain_cost(ch[longest])) longest = c;
+        coop_order.push_back((uint32_t)c);
+        coop_threads_max = std::max(coop_threads_max, coop_threads(ch[c]));
+        coop_lds_max = std::max(coop_lds_max, coop_lds(ch[c]));
     }
-    coop = coop && longest >= 0 &&
-           (o.block_lanes > 1 || (coop_gains(ch[longest]) && coop_waves <= (uint64_t)n_cu * COOP_WAVES));
+    coop = coop && !coop_order.empty();
+    if (coop) {
+        std::stable_sort(coop_order.begin(), coop_order.end(),
+                         [&](uint32_t x, uint32_t y) { return chain_cost(ch[x]) > chain_cost(ch[y]); });
+        if (o.block_lanes == 0) coop = coop_gains(ch[coop_order[0]]);
+    }
+    if (coop) {
+        const void *fn = coop_kernel(fp32);
+        if (int rc = set_lds_attr(fn, coop_lds_max)) return bail(rc);
+        int occ = 0;
+        CREATE_CHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, (int)coop_threads_max, coop_lds_max));
+        if (o.block_lanes == 0) coop = coop_in_time(ch, coop_order, (size_t)occ * n_cu, fp32);
+    }
 
     // internal chain order and bundles (segmented chains last)
     std::vector<DevBundle> bundles[2];
@@ -773,11 +830,7 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
         budget = std::min<size_t>(budget, (size_t)lds_max);
         PackOut p;
         if (coop) {
-            // the longest first: they end last
-            for (int c = 0; c < n_chains; ++c)
-                if (!segS[c]) p.order.push_back((uint32_t)c);
-            std::stable_sort(p.order.begin(), p.order.end(),
-                             [&](uint32_t x, uint32_t y) { return chain_cost(ch[x]) > chain_cost(ch[y]); });
+            p.order = coop_order;
         } else {
             p = pack(e->specs, ch, e->T, budget / 8, (size_t)lds_max / 8 - 64, segS);
         }
@@ -888,15 +941,12 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
         if (coop) {
             Group G;
             G.coop = 1;
+            G.threads = coop_threads_max;
+            G.lds = coop_lds_max;
             std::vector<uint32_t> list;
-            for (int k = 0; k < n_chains; ++k) {
-                if (segS[order[k]]) continue;
-                list.push_back((uint32_t)k);
-                G.threads = std::max(G.threads, coop_threads(e->hch[k]));
-                G.lds = std::max(G.lds, coop_lds(e->hch[k]));
-            }
+            for (int k = 0; k < n_chains; ++k)
+                if (!segS[order[k]]) list.push_back((uint32_t)k);
             G.n_items = G.grid = (uint32_t)list.size();
-            if (int rc = set_lds_attr(coop_kernel(e->form == JMM_FORM_BATCHED_FP32), G.lds)) return bail(rc);
             e->grp.push_back(G);
             Group &Gc = e->grp.back();
             if (int rc = dalloc(&Gc.d_list, Gc.n_items)) return bail(rc);
@@ -920,7 +970,6 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
             // (the larger ones with two waves' registers: 8.6, a CU then
             // holds only one of the others beside them; a smaller share for
             // the others, 40 or 36 KB of 45: 7.37, 7.59).
-            const int fp32 = e->form == JMM_FORM_BATCHED_FP32;
             const bool may3 = !g && e->T == 256 && bv.size() > 2 * (size_t)n_cu;
             const size_t share = (size_t)lds_cu / 3 - BATCHED_STATIC;
             size_t limit = 0, largest = 0;
@@ -999,7 +1048,6 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
             }
         }
         if (!segv.empty()) {
-            const int fp32 = e->form == JMM_FORM_BATCHED_FP32;
             if (o.seg_lanes > 2) return bail(fail(JMM_EINVAL, "jmm_create: seg_lanes must be 0, 1 or 2"));
             e->n_segs = (uint32_t)segv.size();
             e->seg_wgmax = wgmax;
