@@ -284,14 +284,17 @@ static uint64_t chain_cost(const DevChain &c) { return (uint64_t)c.smax * (c.w +
 
 // Whether a chain runs faster with several lanes per block when it has the CU
 // to itself: with more than one partner a side and at least 4 lanes per block
-// (up to 128 blocks), or with two partners a side (2 lanes per block take them
-// at once).  us per sweep, FP32 / FP64: LJ chains (6 partners) of 64 17.2 -> 8.4
-// / 22.6 -> 9.1, of 1000 (128 blocks) 17.5 -> 14.5 / 23.2 -> 15.1, of 4000 (256
-// blocks) 31.0 -> 32.9 / 42.4 -> 41.5; hard rods with a well (1 partner) of 64
-// 4.7 -> 5.4, of 1000 6.9 -> 7.6.
-static bool coop_gains(const DevChain &c)
+// (up to 128 blocks), or, FP64, with two partners a side (2 lanes per block take
+// them at once; the FP32 walk's two partners at a time on one lane are as
+// fast).  us per sweep, FP32 / FP64: LJ chains (6 partners) of 64 17.2 -> 8.4 /
+// 22.6 -> 9.1, of 1000 (128 blocks) 17.5 -> 14.5 / 23.2 -> 15.1, of 4000 (256
+// blocks) 31.0 -> 32.9 / 42.4 -> 41.5; with 2 partners of 400 (128 blocks) 7.2
+// -> 7.2 / 10.3 -> 7.0, of 1000 (256 blocks) 7.9 -> 8.4 / 10.7 -> 9.2, of 2000
+// 12.6 -> 13.3 / 18.5 -> 15.5; hard rods with a well (1 partner) of 64 4.7 ->
+// 5.4, of 1000 6.9 -> 7.6.
+static bool coop_gains(const DevChain &c, bool fp32)
 {
-    return c.w >= 2 && (c.B <= 128 || c.w == 2);
+    return c.w >= 2 && (c.B <= 128 || (c.w == 2 && !fp32));
 }
 
 // Whether chains that are launched one per workgroup, in this order, end
@@ -804,7 +807,7 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
     if (coop) {
         std::stable_sort(coop_order.begin(), coop_order.end(),
                          [&](uint32_t x, uint32_t y) { return chain_cost(ch[x]) > chain_cost(ch[y]); });
-        if (o.block_lanes == 0) coop = coop_gains(ch[coop_order[0]]);
+        if (o.block_lanes == 0) coop = coop_gains(ch[coop_order[0]], fp32);
     }
     if (coop) {
         const void *fn = coop_kernel(fp32);

@@ -59,3 +59,13 @@ def test_chains_that_wait_for_others(gpu, form):
     assert np.array_equal(s0, s1) and np.array_equal(L0, L1) and np.array_equal(U0, U1)
     assert all(np.array_equal(a, b) for a, b in zip(x0, x1))
     assert all(np.array_equal(c0[k], c1[k]) for k in c0)
+
+
+def test_two_partners_a_side(gpu):
+    """Two lanes per block (more than 128 blocks) gain in FP64 only."""
+    for N, fp32, fp64 in ((64, 16, 16), (400, 4, 4), (800, 1, 2), (2000, 1, 2)):
+        ch = Chain(N=N, L0=N / 0.48, T=0.8, P=0.7, boundary=nat.WALLS, ensemble=nat.NPT, max_dv=1.0, max_step=0.1,
+                   nbn=2, seed=9, **lj(cutoff=np.inf, shifted=0))
+        for form, lanes in (("batched_fp32", fp32), ("batched_fp64", fp64)):
+            with Engine([ch], form=form, sample_capacity=1) as e:
+                assert e.layout(0)["lanes"] == lanes, (N, form)
