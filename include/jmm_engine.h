@@ -214,9 +214,13 @@ int jmm_full_energy(jmm_engine *e, double *U_out);
  * 1896-1961): copies every chain's samples since the last read into
  * out[c * max_sweeps + s] and empties the device buffer.  *n_out = sweeps
  * copied per chain (all chains have the same count).  The samples are put
- * in this layout on the device (the first read allocates a staging buffer of
- * sample_capacity x n_chains x 24 bytes, kept until destroy) and arrive in
- * one copy.  Synchronous. */
+ * in this layout on the device: reads of up to 64 KiB straight into a pinned
+ * buffer of that size, larger ones in a staging buffer of sample_capacity x
+ * n_chains x 24 bytes, from which they arrive in one copy (the first read of
+ * either kind allocates its buffer, kept until destroy).  With max_sweeps above
+ * the pending sweeps a larger read also takes host memory of its own size
+ * during the call (without it the rows come in parts); what lies behind the
+ * copied samples of a row is not written.  Synchronous. */
 int jmm_read_samples(jmm_engine *e, jmm_sample *out, uint32_t max_sweeps, uint32_t *n_out);
 
 /* jmm_read_samples plus, for an engine created with sample_virial, the
@@ -233,7 +237,9 @@ int jmm_read_samples_virial(jmm_engine *e, jmm_sample *out, double *virial, uint
  * tight serving loops, harnesses that forbid hipMalloc): the transposition
  * is staged in a fixed 16 MiB device array that the library holds per GPU
  * until the process ends, instead of the buffer jmm_read_samples allocates
- * on first use; no hipMalloc, hipFree or allocating library call is made.
+ * on first use; no hipMalloc, hipFree or allocating library call is made, and
+ * no host memory is allocated (rows of max_sweeps above the pending sweeps come
+ * in parts through 128 KiB of the caller's stack).
  * At most (16 MiB - 4 bytes per chain, rounded up to 256) / 24 bytes of
  * chain-sweeps per call (about 699,000): a larger read is refused with
  * JMM_EINVAL and drains nothing.  Same output, layout and draining as

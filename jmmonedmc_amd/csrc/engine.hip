@@ -1314,23 +1314,34 @@ static unsigned char *stage(jmm_engine *e)
 }
 
 // n_rows rows of row_bytes, contiguous on the device, to rows pitch bytes
-// apart: one contiguous copy (a pitched device-to-host copy goes row by row,
-// measured 6.7 us a row: 27.8 ms of the 37.2 that a block of 100 sweeps of 4096
-// chains took, now 0.6), spread on the host where the pitch is larger.
-static int copy_rows(void *out, size_t pitch, const void *dev, size_t row_bytes, size_t n_rows)
+// apart, nothing between them written.  A pitched device-to-host copy goes row
+// by row, measured 6.7 us a row: 27.8 ms of the 37.2 that a block of 100 sweeps
+// of 4096 chains took; so rows as wide as the pitch are one contiguous copy
+// (0.6 ms), long rows one each (above ROW_BYTES the row's own time exceeds what
+// a second pass on the host would cost), and the others go through a buffer on
+// the host: of the whole read where one may be had (1.0 ms), else of
+// HOST_BYTES on the stack (1.2 ms).
+constexpr size_t ROW_BYTES = size_t(128) << 10, HOST_BYTES = size_t(128) << 10;
+
+static int copy_rows(void *out, size_t pitch, const void *dev, size_t row_bytes, size_t n_rows, bool may_allocate)
 {
     if (pitch == row_bytes || n_rows == 1) {
         HIPCHK(hipMemcpy(out, dev, row_bytes * n_rows, hipMemcpyDeviceToHost));
         return 0;
     }
-    std::unique_ptr<unsigned char[]> tmp(new (std::nothrow) unsigned char[row_bytes * n_rows]);
-    if (!tmp) {
-        HIPCHK(hipMemcpy2D(out, pitch, dev, row_bytes, row_bytes, n_rows, hipMemcpyDeviceToHost));
-        return 0;
+    unsigned char few[HOST_BYTES];
+    std::unique_ptr<unsigned char[]> all;
+    if (may_allocate && row_bytes < ROW_BYTES) all.reset(new (std::nothrow) unsigned char[row_bytes * n_rows]);
+    const size_t step = all ? n_rows : row_bytes < ROW_BYTES ? std::max<size_t>(1, HOST_BYTES / row_bytes) : 1;
+    unsigned char *to = (unsigned char *)out;
+    const unsigned char *from = (const unsigned char *)dev;
+    for (size_t r = 0; r < n_rows; r += step) {
+        const size_t m = std::min(step, n_rows - r);
+        unsigned char *buf = all ? all.get() : m > 1 ? few : to + r * pitch;
+        HIPCHK(hipMemcpy(buf, from + r * row_bytes, row_bytes * m, hipMemcpyDeviceToHost));
+        if (all || m > 1)
+            for (size_t k = 0; k < m; ++k) std::memcpy(to + (r + k) * pitch, buf + k * row_bytes, row_bytes);
     }
-    HIPCHK(hipMemcpy(tmp.get(), dev, row_bytes * n_rows, hipMemcpyDeviceToHost));
-    for (size_t r = 0; r < n_rows; ++r)
-        std::memcpy((unsigned char *)out + r * pitch, tmp.get() + r * row_bytes, row_bytes);
     return 0;
 }
 
@@ -1372,9 +1383,9 @@ int jmm_read_samples_virial(jmm_engine *e, jmm_sample *out, double *virial, uint
                 if (virial) std::memcpy((unsigned char *)virial + c * vpitch, (unsigned char *)pv + c * vrec, vrec);
             }
         } else {
-            if (int rc = copy_rows(out, pitch, ps, rec, (size_t)e->n)) return rc;
+            if (int rc = copy_rows(out, pitch, ps, rec, (size_t)e->n, true)) return rc;
             if (virial)
-                if (int rc = copy_rows(virial, vpitch, pv, vrec, (size_t)e->n)) return rc;
+                if (int rc = copy_rows(virial, vpitch, pv, vrec, (size_t)e->n, true)) return rc;
         }
     }
     *n_out = n;
@@ -1409,7 +1420,7 @@ int jmm_read_samples_noalloc(jmm_engine *e, jmm_sample *out, uint32_t max_sweeps
         HIPCHK(hipStreamSynchronize(e->stream));
         e->write_pos = 0;
         if (int rc = copy_rows(out, (size_t)max_sweeps * sizeof(jmm_sample), d_rec, (size_t)n * sizeof(SampleRec),
-                               (size_t)e->n))
+                               (size_t)e->n, false))
             return rc;
     }
     *n_out = n;
