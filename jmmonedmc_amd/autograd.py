@@ -31,6 +31,9 @@ def _observables(x: torch.Tensor, L: torch.Tensor, chain: Chain, theta, precisio
     x = x.contiguous()
     L = L.contiguous()
     n, N = x.shape
+    # the kernel reads n lengths, one a configuration
+    if n and (L.dim() == 0 or L.shape[0] < n or L.numel() != L.shape[0]):
+        raise ValueError(f"L of shape {tuple(L.shape)} does not hold a length for each of {n} configurations")
     th = [float(t) for t in theta]
     p = list(chain.pot_p) + [0.0] * (4 - len(chain.pot_p))
     p[0], p[1] = th[0], th[1]
