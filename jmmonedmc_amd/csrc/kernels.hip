@@ -2877,6 +2877,8 @@ __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, dou
             active = active && !(d > q.rc);
             if (!__ballot(active)) break;
             const bool in = active && inside64<KIND>(q, d);
+            // a caller's rods may be longer than the well is wide
+            if (KIND == POT_HRSW && active && !in && d < q.p0) acc[0] += INFINITY;
             if (++j == N) {
                 j = 0;
                 off = L;
