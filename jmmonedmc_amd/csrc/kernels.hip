@@ -112,6 +112,11 @@ __device__ __forceinline__ double delta_e32(const Pot &q, const double *X, int64
     return left + right;
 }
 
+__device__ __forceinline__ uint32_t half_of(uint32_t size)
+{
+    return size >= HALF_MIN ? (size + 1) / 2 : size;
+}
+
 // Box-length trial energy over the pairs whose left member is in [p0, p1),
 // for a scaling of every coordinate by sc.  Sets bad when a scaled nearest
 // pair falls inside the hard core.  The energy change pair by pair,
@@ -521,9 +526,17 @@ __device__ __forceinline__ void run_bundle_gx(const SweepArgs &a, const DevBundl
         double vpart = 0.0, upart = 0.0;
         if (npt) {
             vp = vol_propose<sizeof(Real) == 4 && KIND == POT_LJ>(ch, L, sweep);
-            if (vp.valid && act)
-                vpart = scaled_delta<Real, KIND>(q, vp.bk, gmin, X, N, per, L, vp.Lp, vp.sc, w, start,
-                                                 start + size, 1, bad, upart);
+            // long blocks in two halves, as the other placements (half_of)
+            uint32_t p0 = start, p1 = start + half_of(size);
+#pragma unroll 1
+            for (int part = 0; part < 2; ++part) {
+                double u = 0.0;
+                if (vp.valid && p0 < p1)
+                    vpart += scaled_delta<Real, KIND>(q, vp.bk, gmin, X, N, per, L, vp.Lp, vp.sc, w, p0, p1, 1, bad, u);
+                upart += u;
+                p0 = p1;
+                p1 = start + size;
+            }
         }
         {
             double v[3] = {dUs, vpart, upart};
@@ -943,11 +956,6 @@ __device__ __forceinline__ bool trial_lds(const LdsChain &c, const Pot &q, doubl
     dE = KIND == POT_HRSW ? -q.p1 * (double)wL + -q.p1 * (double)wR : sL + sR;
     const float bf = fexp(-betaf * (float)dE);
     return go && (dE <= 0.0 || (double)bf > u);
-}
-
-__device__ __forceinline__ uint32_t half_of(uint32_t size)
-{
-    return size >= HALF_MIN ? (size + 1) / 2 : size;
 }
 
 // Box-length trial (fav, src/jmmMCState.cpp:2161-2293), one lane's share
