@@ -93,10 +93,12 @@ typedef struct jmm_engine_opts {
     uint32_t sample_capacity; /* per-chain sweeps held on device between reads (0 = 1024) */
     uint32_t block_sweeps;    /* sweeps per kernel launch (0 = 100) */
     uint32_t wg_threads;      /* batched forms: lanes per workgroup, rounded up to 256, 512 or
-                                 1024 and to the largest chain's block count (0 = 256) */
+                                 1024 and to the largest chain's block count (0 = 256);
+                                 not used with several lanes per block (block_lanes) */
     uint32_t use_graph;       /* 1: replay sweep blocks from a captured hipGraph */
     uint32_t log_accepts;     /* 1: record one byte per displacement trial (tests) */
-    uint32_t lds_budget;      /* batched forms: LDS bytes per workgroup (0 = 64 KiB) */
+    uint32_t lds_budget;      /* batched forms: LDS bytes per workgroup (0 = 64 KiB); not used
+                                 with several lanes per block (block_lanes) */
     uint32_t seg_lds;         /* batched forms: a chain whose LDS image exceeds this many bytes
                                  (0 = the device's LDS per workgroup) is split into segments of
                                  consecutive blocks, one workgroup each, neighbours
@@ -110,10 +112,11 @@ typedef struct jmm_engine_opts {
     uint32_t sample_virial;   /* 1: after every sweep each chain's virial W = sum -d phi'(d)
                                  and hypervirial sum -d W'(d) are computed (FP64) and kept
                                  with the samples (jmm_read_samples_virial) */
-    uint32_t block_lanes;     /* batched forms, chains that are not split: 0 = chosen by the
-                                 number of chains, 1 = one lane per block of particles, 2 or
-                                 more = several (a workgroup per chain) where every chain's
-                                 window allows it; results are the same bits either way */
+    uint32_t block_lanes;     /* batched forms, chains that are not split: 0 = several where the
+                                 engine expects them to be faster (few chains), 1 = one lane
+                                 per block of particles, 2 or more = several (a workgroup per
+                                 chain) where every chain's window and block count allow it;
+                                 results are the same bits either way */
 } jmm_engine_opts;
 
 /* One per chain per sweep (the per-sweep form of the reference's per-trial
@@ -164,7 +167,8 @@ typedef struct jmm_layout {
     uint32_t mode;       /* JMM_MODE_* */
     uint32_t segments;   /* workgroups the chain spans (1 unless split) */
     uint64_t lds_bytes;  /* LDS image of the chain, or of one segment when split */
-    uint32_t lanes;      /* lanes per block (2 when split chains share trials over two lanes) */
+    uint32_t lanes;      /* lanes per block (2 when split chains share trials over two lanes; 2,
+                            4 or 16 when a chain has a workgroup with several) */
     uint32_t reserved;
 } jmm_layout;
 

@@ -13,7 +13,9 @@ admit chains of up to that many blocks and put more blocks in one; 1024
 lanes cap the kernel at 128 VGPRs, so they spill),
 whether sweep blocks replay a captured hipGraph, and, for chains too large
 for one workgroup's LDS, the split threshold (how many workgroups share a
-chain) and the lanes per block of a split chain (1 or 2).  Results can be
+chain) and the lanes per block of a split chain (1 or 2).  tune() adds the
+lanes per block of the other chains (lane_candidates); engines that take
+several do not use the LDS budget and the width.  Results can be
 cached in a JSON file keyed by a signature of the chain mix and the device.
 """
 from __future__ import annotations
@@ -46,8 +48,10 @@ SPLIT_CANDIDATE_BYTES = 96 * 1024
 def candidates_for(chains) -> list:
     """DEFAULT_CANDIDATES, the 512- and 1024-lane workgroups at two LDS
     budgets each, and,
-    when a chain may be split, split thresholds of 64 and 32 KiB per
-    workgroup and two lanes per block of a split chain."""
+    when a chain may be split, one and two lanes per block of a split chain
+    at the default split threshold and at 64 and 32 KiB per workgroup (two
+    lanes ask for more of the CUs, so a batch may be refused with them and
+    not with one)."""
     cands = [dict(c) for c in DEFAULT_CANDIDATES]
     cands += [dict(lds_budget=65536, wg_threads=512, use_graph=True),
               dict(lds_budget=98304, wg_threads=512, use_graph=True),
@@ -55,8 +59,17 @@ def candidates_for(chains) -> list:
               dict(lds_budget=98304, wg_threads=1024, use_graph=True)]
     if any(8 * c.N > SPLIT_CANDIDATE_BYTES for c in chains):
         base = dict(lds_budget=65536, wg_threads=256, use_graph=True)
-        cands += [dict(base, seg_lanes=2), dict(base, seg_lds=65536), dict(base, seg_lds=32768)]
+        cands += [dict(base, seg_lanes=lanes, **thr) for thr in ({}, dict(seg_lds=65536), dict(seg_lds=32768))
+                  for lanes in (1, 2)]
     return cands
+
+
+def lane_candidates() -> list:
+    """One and several lanes per block of the chains that are not split,
+    whatever the engine would take by itself (where several are not possible
+    the second is the first again)."""
+    base = dict(lds_budget=65536, wg_threads=256, use_graph=True)
+    return [dict(base, block_lanes=1), dict(base, block_lanes=2)]
 
 
 @dataclass
@@ -93,7 +106,7 @@ def tune(chains, form: str = "batched_fp32", candidates=None, block_sweeps: int 
         if sig in stored:
             r = stored[sig]
             return TuneResult(best=r["best"], ms_per_sweep=r["ms_per_sweep"], signature=sig)
-    cands = candidates or candidates_for(chains)
+    cands = candidates or candidates_for(chains) + lane_candidates()
     times = {}
     for c in cands:
         opts = dict(c)
