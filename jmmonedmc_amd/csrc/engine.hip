@@ -297,17 +297,36 @@ static bool coop_gains(const DevChain &c, bool fp32)
     return c.w >= 2 && (c.B <= 128 || (c.w == 2 && !fp32));
 }
 
+// us per sweep of a chain by itself, from its phases: fits to hard-rod and LJ
+// chains (1 to 8 partners a side) of 2 to 256 blocks of 9 to 128, NPT.  With
+// several lanes per block: the upper end over the windows (16 lanes 0.40 to 0.58
+// a phase with up to two waves, 0.49 to 0.72 with eight; 4 lanes 0.64 to 1.06
+// and 0.77 to 1.45); with one lane: the lower end over the block counts.
+static double coop_time(const DevChain &c, bool fp32)
+{
+    const double waves = coop_threads(c) / 64;
+    const uint32_t lanes = coop_lanes(c.B);
+    const double phase = lanes == 16 ? (fp32 ? 0.55 + 0.02 * waves : 0.62 + 0.04 * waves)
+                       : lanes == 4  ? (fp32 ? 0.67 + 0.1 * waves : 0.85 + 0.1 * waves)
+                                     : (fp32 ? 2.55 : 2.7);
+    return 4.5 + phase * c.smax;
+}
+
+static double one_lane_time(const DevChain &c, bool fp32)
+{
+    static const double phase[2][COOP_W + 1] = {{0.93, 0.93, 1.56, 1.66, 1.94, 2.1, 2.28, 2.5, 2.72},
+                                                {0.82, 0.82, 1.22, 1.22, 1.45, 1.5, 1.65, 1.7, 1.72}};
+    return 3.0 + phase[fp32 ? 1 : 0][std::min(c.w, COOP_W)] * c.smax;
+}
+
 // Whether chains that are launched one per workgroup, in this order, end
 // before they would with one lane per block.  All resident at once (the launch
 // gives every workgroup the lanes and the LDS of the largest chain, so `slots`
 // of them): yes, where the longest gains (coop_gains).  Otherwise the later
 // ones wait for the earlier, while with one lane every chain runs at once: the
 // launch's end is taken from the chains' estimated times, each on the slot that
-// is free first, and compared with the longest chain's on one lane.  The
-// estimates, us per sweep, are fits to LJ and hard-rod chains of 25 to 1000:
-// 0.05 (cost + 100) with several lanes (times 1.04 to 1.5 for 1 to 8 waves at
-// 16 lanes per block, 1.8 at 4, 2.5 at 2), 0.225 (FP64 0.295) (cost + 16) with
-// one.  Measured, one lane -> several, FP32 / FP64 (taken where marked *):
+// is free first, and compared with the longest chain's on one lane.  Measured,
+// us per sweep, one lane -> several, FP32 / FP64 (taken where marked *):
 //   log-uniform 20 to 256, LJ and rods, 300 chains  28.9 -> 11.4* / 37.5 -> 12.7*
 //                                       600         28.5 -> 20.2* / 37.5 -> 22.6*
 //                                      1500         28.6 -> 44.9  / 37.6 -> 50.4
@@ -315,21 +334,16 @@ static bool coop_gains(const DevChain &c, bool fp32)
 //   1000 of 25 beside one of 300                    27.0 -> 40.8  / 35.2 -> 45.8
 //   1024 of 64 (all resident)                       18.2 -> 10.1* / 23.4 -> 11.8*
 //   257 of 250 (256 resident)                       18.0 -> 20.3  / 23.5 -> 23.3
+//   700 of 3000 to 8000 in 64 blocks (256 resident) 217  -> 270   / 290  -> 292
 static bool coop_in_time(const std::vector<DevChain> &ch, const std::vector<uint32_t> &order, size_t slots, bool fp32)
 {
     if (order.size() <= slots) return true;
     if (!slots) return false;
-    auto several = [&](const DevChain &c) {
-        const double waves = coop_threads(c) / 64, lanes = coop_lanes(c.B);
-        const double f = lanes == 16 ? (fp32 ? 1.0 + 0.04 * waves : 1.05 + 0.055 * waves)
-                       : lanes == 4  ? (fp32 ? 1.75 : 1.85)
-                                     : 2.5;
-        return 0.05 * (double)(chain_cost(c) + 100) * f;
-    };
     double limit = 0.0, work = 0.0;
     for (uint32_t c : order) {
-        limit = std::max(limit, 0.95 * (fp32 ? 0.225 : 0.295) * (double)(chain_cost(ch[c]) + 16));
-        work += several(ch[c]);
+        // (the estimates lie at the far ends of their fits: 10 % apart)
+        limit = std::max(limit, 1.08 * one_lane_time(ch[c], fp32));
+        work += coop_time(ch[c], fp32);
     }
     if (work > limit * (double)slots) return false;
     std::priority_queue<double, std::vector<double>, std::greater<double>> ends;
@@ -339,7 +353,7 @@ static bool coop_in_time(const std::vector<DevChain> &ch, const std::vector<uint
             start = ends.top();
             ends.pop();
         }
-        const double end = start + several(ch[c]);
+        const double end = start + coop_time(ch[c], fp32);
         if (end > limit) return false;
         ends.push(end);
     }

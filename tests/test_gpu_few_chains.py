@@ -12,9 +12,9 @@ from helpers import hrsw, lj
 pytestmark = pytest.mark.gpu
 
 
-def npt(N, c, pot=None):
+def npt(N, c, pot=None, bcap=256):
     return Chain(N=N, L0=max(N / 0.4, 9.0), T=1.0, P=0.5, ensemble=nat.NPT, max_dv=0.01, seed=7, chain_id=c, eci=3,
-                 **(pot or lj()))
+                 bcap=bcap, **(pot or lj()))
 
 
 def uneven(n, pots):
@@ -33,6 +33,7 @@ CASES = {
     "one_long_among_many": (lambda: [npt(25, c) for c in range(1000)] + [npt(300, 1000)], False, False),
     "one_block_chains": (lambda: [npt(13, c) for c in range(2000)] + [npt(300, 2000)], False, False),
     "uneven_300": (lambda: uneven(300, [hrsw, lj]), True, True),
+    "long_blocks": (lambda: [npt(3000 + 7 * c, c, bcap=64) for c in range(700)], False, False),
     "uneven_1500": (lambda: uneven(1500, [hrsw, lj]), False, False),
 }
 
