@@ -987,7 +987,17 @@ int jmm_create(const jmm_chain_spec *specs, int n_chains, const jmm_engine_opts 
             // (the larger ones with two waves' registers: 8.6, a CU then
             // holds only one of the others beside them; a smaller share for
             // the others, 40 or 36 KB of 45: 7.37, 7.59).
-            const bool may3 = !g && e->T == 256 && bv.size() > 2 * (size_t)n_cu;
+            // The third wave shortens the queue, not the longest bundle: in the
+            // FP64 form, whose waves it slows by 3 to 4 %, it is left out where
+            // the longest alone takes longer than some 0.7 of the others' share
+            // (FP64, three waves against two, us a sweep: 1500 hard-rod chains of
+            // 20 to 8000, 0.5 of it, 36.0 and 34.8; 800 of 1000 to 8000, 0.66,
+            // 36.2 and 35.0; 2200 of 20 to 8000, 0.74, 36.8 and 38.2, 3000, 1.0,
+            // 43 and 53; FP32, 1500: 32.1 and 31.8).
+            double work = 0.0;
+            for (auto &b : bv) work += bundle_cost(b, e->hch, slots);
+            const bool queues = fp32 || work >= 0.7 * 2 * n_cu * bundle_cost(bv.front(), e->hch, slots);
+            const bool may3 = !g && e->T == 256 && bv.size() > 2 * (size_t)n_cu && queues;
             const size_t share = (size_t)lds_cu / 3 - BATCHED_STATIC;
             size_t limit = 0, largest = 0;
             for (auto &b : bv) largest = std::max<size_t>(largest, b.lds_doubles * sizeof(double));
