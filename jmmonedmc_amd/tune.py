@@ -13,9 +13,10 @@ admit chains of up to that many blocks and put more blocks in one; 1024
 lanes cap the kernel at 128 VGPRs, so they spill),
 whether sweep blocks replay a captured hipGraph, and, for chains too large
 for one workgroup's LDS, the split threshold (how many workgroups share a
-chain) and the lanes per block of a split chain (1 or 2).  tune() adds the
-lanes per block of the other chains (lane_candidates); engines that take
-several do not use the LDS budget and the width.  Results can be
+chain) and the lanes per block of a split chain (1 or 2).  The lanes per
+block of the other chains are the engine's own choice, which these candidates
+leave alone; lane_candidates() fixes them (engines that take several do not
+use the LDS budget and the width).  Results can be
 cached in a JSON file keyed by a signature of the chain mix and the device.
 """
 from __future__ import annotations
@@ -67,7 +68,8 @@ def candidates_for(chains) -> list:
 def lane_candidates() -> list:
     """One and several lanes per block of the chains that are not split,
     whatever the engine would take by itself (where several are not possible
-    the second is the first again)."""
+    the second is the first again); for
+    tune(chains, candidates=candidates_for(chains) + lane_candidates())."""
     base = dict(lds_budget=65536, wg_threads=256, use_graph=True)
     return [dict(base, block_lanes=1), dict(base, block_lanes=2)]
 
@@ -106,7 +108,7 @@ def tune(chains, form: str = "batched_fp32", candidates=None, block_sweeps: int 
         if sig in stored:
             r = stored[sig]
             return TuneResult(best=r["best"], ms_per_sweep=r["ms_per_sweep"], signature=sig)
-    cands = candidates or candidates_for(chains) + lane_candidates()
+    cands = candidates or candidates_for(chains)
     times = {}
     for c in cands:
         opts = dict(c)

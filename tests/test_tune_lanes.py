@@ -40,7 +40,7 @@ def test_block_lanes_are_timed(monkeypatch):
             return 1, self.ms, 1
 
     monkeypatch.setattr(t, "Engine", Fake)
-    res = t.tune(configs.c5(2))
+    res = t.tune(configs.c5(2), candidates=t.candidates_for(configs.c5(2)) + t.lane_candidates())
     assert {o.get("block_lanes") for o in seen} == {None, 1, 2}
     assert res.best["block_lanes"] == 1
     assert len(seen) == len({str(sorted(o.items())) for o in seen})
