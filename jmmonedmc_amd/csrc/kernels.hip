@@ -1411,7 +1411,7 @@ __device__ __forceinline__ void run_bundle_lds(const SweepArgs &a, const DevBund
 // (all potentials together, longest first) until it is empty; all waves of a
 // workgroup leave together when the queue is drained.  The potential is
 // uniform per bundle.  W waves per SIMD bound the registers: 2 (256, 193 used),
-// or 3 for 256 lanes (168, 21 spilled outside the phases), which hides more of
+// or 3 for 256 lanes (168; 9 spilled in FP32, 1 in FP64, outside the phases), which hides more of
 // the phases' latency where there are bundles for it: 4096 mixed chains of 32 to
 // 4000, FP32, 55.0 us a sweep with 2, 44.6 with 3 (4: 128 registers, 269
 // spilled, 59.5); bundles that fit at 2 lose 1 to 2 % to the spills.
@@ -2846,7 +2846,8 @@ struct ObsScratch {
 // waves, whatever the workgroup has.
 // The kernel, FP32: 64 Yukawa configurations of 65,536 314 us with both sides
 // walked, 244 with each pair once, 225 with the divisions of pair_obs_f and
-// tiles of 512; 1024 LJ chains of 1024 28 and 22 us.
+// tiles of 512 (back to back and with k_obs_sum 210); 1024 LJ chains of 1024 28
+// and 22 us.
 template <typename Real, int KIND>
 __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, double L, double sc, uint32_t p0,
                                         uint32_t p1, double *out, double *grad, ObsScratch &sm)
