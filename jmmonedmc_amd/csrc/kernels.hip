@@ -2846,7 +2846,7 @@ struct ObsScratch {
 // waves, whatever the workgroup has.
 // The kernel, FP32: 64 Yukawa configurations of 65,536 314 us with both sides
 // walked, 244 with each pair once, 225 with the divisions of pair_obs_f and
-// tiles of 512 (back to back and with k_obs_sum 210); 1024 LJ chains of 1024 28
+// tiles of 512 (back to back and with k_obs_sum 212); 1024 LJ chains of 1024 28
 // and 22 us.
 template <typename Real, int KIND>
 __device__ __forceinline__ void run_obs(const DevChain &ch, const double *X, double L, double sc, uint32_t p0,
